@@ -183,12 +183,12 @@ def table_eval_fn(lib, table, src, srcdesc, outs, descs, stream):
 
 
 def kernel_labels(nw, lc):
-    return {"rec_g8": f"k_stencils_rec<{nw},{lc},8>", "rec_g4": f"k_stencils_rec<{nw},{lc},4>",
-            "rec_g16": f"k_stencils_rec<{nw},{lc},16>",
-            "split": f"k_stencils_sliced<{nw},{lc}>", "csr_lds": f"k_stencils_csr<{nw},{lc}>",
+    compact = f"k_stencils_compact<{nw},{lc}>"
+    return {"far_order": compact, "split": f"k_stencils_sliced<{nw},{lc}>",
+            "csr_lds": f"k_stencils_csr<{nw},{lc}>",
             "rec_pair": f"k_stencils_rec_paired<{lc},16>",
-            "tiled8": f"k_stencils_tiled<{nw},{lc},8>", "tiled4": f"k_stencils_tiled<{nw},{lc},4>",
-            "tiled4_dom": f"k_stencils_tiled<{nw},{lc},4> (rows by dominant vertex only)"}
+            "tiled": f"{compact} (rows by dominant vertex, size windows)",
+            "tiled_dom": f"{compact} (rows by dominant vertex only)"}
 
 
 def bbox_rel_err(x, ref):
@@ -228,15 +228,14 @@ def run_stencils(args, lib, name, table_np, src_np, nw, kernel_label, with_cpu, 
     d_src = torch.from_numpy(np.ascontiguousarray(src_np)).to("cuda")
     outs = [torch.empty(n * L, dtype=torch.float32, device="cuda") for _ in range(nw)]
     alg = stencil_bytes(n, nnz, nw, L, src_np.shape[0], nw)
-    # autotune: a few untimed launches of each kernel variant (record slices
-    # with gather groups of 16 / 8 / 4, split-stream slices, CSR with LDS
-    # staging, locality-ordered slices with control points staged in LDS,
-    # and for one weight array paired records; per-table options),
+    # autotune: a few untimed launches of each kernel variant (compact slices
+    # in Far's row order or a locality order, split-stream slices, CSR with
+    # LDS staging, and for one weight array paired records; per-table
+    # options),
     # then the timed region runs exactly `steps` launches of the fastest
     # (layout, group, kernel, layout-2 row order)
-    VARIANTS = {"rec_g8": (0, 8, 0, 0), "rec_g4": (0, 4, 0, 0), "rec_g16": (0, 16, 0, 0),
-                "split": (1, 8, 0, 0), "csr_lds": (0, 8, 1, 0), "tiled8": (2, 8, 0, 0),
-                "tiled4": (2, 4, 0, 0), "tiled4_dom": (2, 4, 0, 2)}
+    VARIANTS = {"far_order": (0, 8, 0, 0), "split": (1, 8, 0, 0), "csr_lds": (0, 8, 1, 0),
+                "tiled": (2, 8, 0, 0), "tiled_dom": (2, 8, 0, 2)}
     if nw == 1:
         VARIANTS["rec_pair"] = (3, 16, 0, 0)
     if args.variant:                      # one variant only (profiling runs)
@@ -781,7 +780,7 @@ def run_batched(args, lib, device, copy_gbps=None):
                      "traffic": tr.get("bytes_per_step") if tr else None,
                      "copy_rate_GBps": copy_gbps,
                      "frac_of_copy_rate": achieved / copy_gbps if copy_gbps else None,
-                     "kernel": "one step: k_batch_stencils_tiled (phase A) + k_batch_patches* "
+                     "kernel": "one step: k_batch_stencils (phase A) + k_batch_patches* "
                                "(phase B), graph launches of every stage",
                      "algorithmic_bytes": alg, "kernel_ms": kms,
                      "output_bytes": out_bytes,
@@ -1071,7 +1070,7 @@ def main():
                     help="cfg3: batch knobs key=value,... set before (or instead of) tuning")
     ap.add_argument("--no-tune", action="store_true", help="cfg3: skip the autotuner")
     ap.add_argument("--variant", default=None,
-                    help="cfg1 / cfg1_refine: time this table variant only (e.g. tiled4)")
+                    help="cfg1 / cfg1_refine: time this table variant only (e.g. tiled)")
     ap.add_argument("--no-parity", action="store_true", help="cfg3: skip the parity checks")
     ap.add_argument("--no-plain", action="store_true",
                     help="cfg3: skip timing the one-mesh-per-launch path")

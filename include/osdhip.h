@@ -130,20 +130,22 @@ osdhip_stencil_table *osdhip_stencil_table_create(int numStencils, const int *si
 /* How a table is laid out on the device and evaluated.  Everything is fixed
  * per table (nothing process-wide), so tables built with different options
  * can be used concurrently.  Results are the same bits whatever the options.
- *   layout:  0 = one interleaved record {index, weights} per entry in 64-row
- *            slices (default); 1 = index and weights in separate streams;
- *            2 = locality-ordered slices: rows grouped by their dominant
- *            control vertex (see order), each slice's distinct control
- *            vertices staged in LDS (for multi-frame batches and large
- *            refinement tables);
+ *   layout:  0 = compact 64-row slices in Far's row order (default): a slice
+ *            lists its distinct control vertices (up to 255), which are
+ *            staged in LDS, and its entries hold one-byte list positions;
+ *            1 = index and weights in separate streams; 2 = compact slices
+ *            in a locality order: rows grouped by their dominant control
+ *            vertex (see order), lists of up to 63 (for multi-frame batches
+ *            and large refinement tables);
  *            3 = paired records for tables of one weight array: a row's
  *            entries 2p and 2p + 1 side by side, read with one 16-byte load
  *            (NULL for tables of 3 or 6 weight arrays; not for batches).
  *   keepCsr: 1 (default) = the Far CSR arrays stay on the device
  *            (osdhip_stencil_table_csr, the CSR kernel); 0 = only the slice
  *            layout is kept (the CSR getters return NULL).
- *   group:   entries per gather group of the slice kernels: 4, 8 (default)
- *            or 16 (layout 2 uses 4, or 8 for 8 and 16).
+ *   group:   entries per gather group of layout 3's kernel: 4, 8 (default)
+ *            or 16 (accepted and kept for the other layouts, whose kernels
+ *            have one group size).
  *   kernel:  osdhip_stencil_table_eval kernel: 0 = slice layout (default),
  *            1 = CSR with LDS staging (needs keepCsr).
  *   order:   layout 2's row order: 0 = by dominant control vertex, then
@@ -152,11 +154,12 @@ osdhip_stencil_table *osdhip_stencil_table_create(int numStencils, const int *si
  *            listing their control vertices (default: the fewest entries
  *            streamed per evaluation); 2 = by dominant control vertex only
  *            (the fewest control vertices per slice: for many-frame
- *            batches, which re-read records from cache but stage control
- *            vertices per frame chunk); 1 = Far's row order (a slice's
- *            outputs are 64 consecutive rows; slices with more distinct
- *            control vertices than the LDS list holds gather them from
- *            memory). */
+ *            batches, which stage control vertices per frame chunk), or
+ *            Far's order for tables of 65,536 rows and more whose slices in
+ *            that order list at most one control vertex per two rows (a
+ *            batch's outputs then leave the caches, and consecutive rows
+ *            write faster); 1 = Far's row order (a slice's outputs are 64
+ *            consecutive rows; lists of up to 255). */
 typedef struct {
     int layout;
     int keepCsr;
@@ -187,12 +190,12 @@ int osdhip_stencil_table_info(const osdhip_stencil_table *table, int *numStencil
                               long long *numEntries, int *numWeightArrays,
                               long long *deviceBytes);
 /* The table's device layout: layout (see osdhip_table_options), number of
- * 64-row slices and, for layout 2, the slices whose control vertices are
- * staged in LDS and the total length of their control lists.  No
+ * 64-row slices and, for layouts 0 and 2, the slices whose control vertices
+ * are staged in LDS and the total length of their control lists.  No
  * counterpart in the reference: a diagnostic of this library's layouts. */
 int osdhip_stencil_table_layout(const osdhip_stencil_table *table, int *layout, int *numSlices,
                                 int *listedSlices, long long *listEntries);
-/* Record entries the table's slices hold (64 x the widest row of every
+/* Entries the table's slices hold (64 x the widest row of every
  * slice: the entries each evaluation streams, padding included) and, for
  * layout 2 with rows by dominant vertex, the window (0, 128 or 512 rows)
  * within which rows were regrouped by size to make a slice's rows alike.
@@ -455,9 +458,9 @@ int osdhip_batch_num_stages(const osdhip_batch *batch);
 int osdhip_batch_run_plain(osdhip_batch *batch, void *stream);
 int osdhip_batch_run_plain_stage(osdhip_batch *batch, int stage, void *stream);
 /* Variant knobs: "a_frames" x "a_group" (frames per chunk, gather group;
- * layout-0 tables: {1x4, 1x8, 2x4, 4x2} or a_frames 0 = a slice's records
- * stay in registers for all frames; layout-2 tables: {1, 2, 4} x {4, 8};
- * other pairs make launches return OSDHIP_ERR_UNSUPPORTED),
+ * layout-0 tables: {1x4, 1x8, 2x4, 4x2} or a_frames 0, which means 4;
+ * layout-2 tables: {1, 2, 4} x {4, 8}; other pairs make launches return
+ * OSDHIP_ERR_UNSUPPORTED; the group changes nothing else),
  * "a_item_slices" (64-row slices per work item), "a_persistent" /
  * "b_persistent" (0 = one block per item, 1 = fixed grid claiming items
  * from a device counter), "b_frames" in {1, 2, 4}, "b_stage" (1 = waves

@@ -5,7 +5,7 @@ Segments reference device buffers (torch tensors) and HipStencilTables; the
 Batch keeps them alive for its own lifetime.
 
 Stencil segment (dict):
-    table   HipStencilTable with one weight array (record layout)
+    table   HipStencilTable with one weight array (layout 0 or 2)
     src     device tensor; element (v, f, k) at src + v*src_v + f*src_f + k
     dst     device tensor; element (row, f, k) at dst + row*dst_v + f*dst_f + k
     frames, src_v, src_f, dst_v, dst_f

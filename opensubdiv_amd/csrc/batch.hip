@@ -59,89 +59,36 @@ struct osdhip_batch {
 
 namespace {
 
-template <int LC, int FC, int G>
-void launchA(const BatchArgs &a, int grid, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_batch_stencils<LC, FC, G>), dim3(grid), dim3(kBlock), 0, st, a);
-}
-
-template <int FC, int G>
+template <int FC>
 bool launchA_lc(int lc, const BatchArgs &a, int grid, hipStream_t st)
 {
     switch (lc) {
-    case 1: launchA<1, FC, G>(a, grid, st); return true;
-    case 2: launchA<2, FC, G>(a, grid, st); return true;
-    case 3: launchA<3, FC, G>(a, grid, st); return true;
-    case 4: launchA<4, FC, G>(a, grid, st); return true;
-    case 5: launchA<5, FC, G>(a, grid, st); return true;
-    case 6: launchA<6, FC, G>(a, grid, st); return true;
-    case 7: launchA<7, FC, G>(a, grid, st); return true;
-    case 8: launchA<8, FC, G>(a, grid, st); return true;
+    case 1: hipLaunchKernelGGL((k_batch_stencils<1, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
+    case 2: hipLaunchKernelGGL((k_batch_stencils<2, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
+    case 3: hipLaunchKernelGGL((k_batch_stencils<3, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
+    case 4: hipLaunchKernelGGL((k_batch_stencils<4, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
+    case 5: hipLaunchKernelGGL((k_batch_stencils<5, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
+    case 6: hipLaunchKernelGGL((k_batch_stencils<6, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
+    case 7: hipLaunchKernelGGL((k_batch_stencils<7, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
+    case 8: hipLaunchKernelGGL((k_batch_stencils<8, FC>), dim3(grid), dim3(kBlock), 0, st, a); return true;
     default: return false;
     }
 }
 
-template <int LC>
-void launchRR(const BatchArgs &a, int grid, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_batch_stencils_rr<LC>), dim3(grid), dim3(kBlock), 0, st, a);
-}
-
-bool launchRR_lc(int lc, const BatchArgs &a, int grid, hipStream_t st)
-{
-    switch (lc) {
-    case 1: launchRR<1>(a, grid, st); return true;
-    case 2: launchRR<2>(a, grid, st); return true;
-    case 3: launchRR<3>(a, grid, st); return true;
-    case 4: launchRR<4>(a, grid, st); return true;
-    case 5: launchRR<5>(a, grid, st); return true;
-    case 6: launchRR<6>(a, grid, st); return true;
-    case 7: launchRR<7>(a, grid, st); return true;
-    case 8: launchRR<8>(a, grid, st); return true;
-    default: return false;
-    }
-}
-
-template <int FC, int G>
-bool launchT_lc(int lc, const BatchArgs &a, int grid, hipStream_t st)
-{
-    switch (lc) {
-    case 1: hipLaunchKernelGGL((k_batch_stencils_tiled<1, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    case 2: hipLaunchKernelGGL((k_batch_stencils_tiled<2, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    case 3: hipLaunchKernelGGL((k_batch_stencils_tiled<3, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    case 4: hipLaunchKernelGGL((k_batch_stencils_tiled<4, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    case 5: hipLaunchKernelGGL((k_batch_stencils_tiled<5, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    case 6: hipLaunchKernelGGL((k_batch_stencils_tiled<6, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    case 7: hipLaunchKernelGGL((k_batch_stencils_tiled<7, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    case 8: hipLaunchKernelGGL((k_batch_stencils_tiled<8, FC, G>), dim3(grid), dim3(kBlock), 0, st, a); return true;
-    default: return false;
-    }
-}
-
-// phase A variants on locality-ordered tables: (frames per chunk, group)
-bool launchT_variant(int lc, int fc, int g, const BatchArgs &a, int grid, hipStream_t st)
-{
-    if (fc == 1 && g == 4) return launchT_lc<1, 4>(lc, a, grid, st);
-    if (fc == 1 && g == 8) return launchT_lc<1, 8>(lc, a, grid, st);
-    if (fc == 2 && g == 4) return launchT_lc<2, 4>(lc, a, grid, st);
-    if (fc == 2 && g == 8) return launchT_lc<2, 8>(lc, a, grid, st);
-    if (fc == 4 && g == 4) return launchT_lc<4, 4>(lc, a, grid, st);
-    if (fc == 4 && g == 8) return launchT_lc<4, 8>(lc, a, grid, st);
-    return false;
-}
-
-// phase A variants: (frames per chunk, gather group); frames 0 = the
-// records of a slice stay in registers for all frames (group ignored)
+// phase A variants: frames per chunk x gather group.  Both slice layouts
+// run the same kernels, which hold a slice's entries in registers whatever
+// the group; the pairs each layout has always accepted are kept (frames 0:
+// every frame's entries from registers, now what every variant does).
 bool launchA_variant(bool tiled, int lc, int fc, int g, const BatchArgs &a, int grid,
                      hipStream_t st)
 {
-    if (tiled) return launchT_variant(lc, fc, g, a, grid, st);
-    if (fc == 0) return launchRR_lc(lc, a, grid, st);
-    if (fc == 1 && g == 4) return launchA_lc<1, 4>(lc, a, grid, st);
-    if (fc == 1 && g == 8) return launchA_lc<1, 8>(lc, a, grid, st);
-    if (fc == 2 && g == 4) return launchA_lc<2, 4>(lc, a, grid, st);
-    if (fc == 4 && g == 2) return launchA_lc<4, 2>(lc, a, grid, st);
-    return false;
+    const bool known = tiled ? (fc == 1 || fc == 2 || fc == 4) && (g == 4 || g == 8)
+                             : fc == 0 || (fc == 1 && (g == 4 || g == 8)) || (fc == 2 && g == 4) ||
+                                   (fc == 4 && g == 2);
+    if (!known) return false;
+    if (fc == 1) return launchA_lc<1>(lc, a, grid, st);
+    if (fc == 2) return launchA_lc<2>(lc, a, grid, st);
+    return launchA_lc<4>(lc, a, grid, st);
 }
 
 // Phase-B launch kinds, each over its own item list: every regular-interior
@@ -449,12 +396,8 @@ static osdhip_batch *batch_create(int length, int numStencilSegments,
         BatchStencilSeg g;
         std::memset(&g, 0, sizeof(g));
         g.rec = t->rec;
-        g.sliceOff = t->sliceOff;
-        g.sliceWidth = t->sliceWidth;
-        g.rowSize = t->rowSize;
+        g.slices = t->slices;
         g.perm = t->perm;
-        g.nuniq = t->nuniq;
-        g.ctrlOff = t->ctrlOff;
         g.ctrl = t->ctrl;
         g.src = s.src;
         g.srcV = s.srcVertexStride;
@@ -950,12 +893,8 @@ int osdhip_batch_epoch(int length, int numStencilSegments, const osdhip_batch_st
         BatchStencilSeg g;
         std::memset(&g, 0, sizeof(g));
         g.rec = t->rec;
-        g.sliceOff = t->sliceOff;
-        g.sliceWidth = t->sliceWidth;
-        g.rowSize = t->rowSize;
+        g.slices = t->slices;
         g.perm = t->perm;
-        g.nuniq = t->nuniq;
-        g.ctrlOff = t->ctrlOff;
         g.ctrl = t->ctrl;
         g.src = s.src;
         g.srcV = s.srcVertexStride;

@@ -1,8 +1,8 @@
 // Batched evaluation: many meshes, each with many frames of control points,
 // in one graph launch of two kernels.
 //
-//   phase A  k_batch_stencils  every stencil segment (one record-layout
-//                              table applied to F frames): refinement
+//   phase A  k_batch_stencils  every stencil segment (one table in compact
+//                              slices applied to F frames): refinement
 //                              tables and the patch-point tables that fill
 //                              each mesh's vertex buffer [control | points];
 //   phase B  k_batch_patches   every patch segment (one mesh's PatchCoords
@@ -10,8 +10,7 @@
 //                              vertex buffers phase A completed.
 //
 // Frames are extra right-hand-side columns: a wave loads a table slice's
-// records once per chunk of FC frames (later chunks hit L1/L2), and a
-// PatchCoord's basis is evaluated once for all frames.  Element (v, f, k)
+// entries once for all frames, and a PatchCoord's basis is evaluated once for all frames.  Element (v, f, k)
 // of a multi-frame buffer lives at base + v * vStride + f * fStride + k, so
 // both frame-major and vertex-major (frames interleaved) layouts work.
 //
@@ -23,25 +22,22 @@
 // item count.
 //
 // Every sum accumulates w * x in the same order as the single-mesh kernels
-// (k_stencils_rec / k_patches), so batched results equal one-mesh-per-launch
+// (k_stencils_compact / k_patches), so batched results equal one-mesh-per-launch
 // results bit for bit.
 #pragma once
+#include <type_traits>
+
 #include "../../include/osdhip.h"
 #include "common.h"
 #include "patch_basis_device.h"
-#include "stencil_sliced.h"
-#include "stencil_tiled.h"
+#include "stencil_compact.h"
 
 namespace osdhip {
 
 struct BatchStencilSeg {
-    const unsigned *rec;          // record layout, one weight array (R = 2)
-    const long long *sliceOff;
-    const int *sliceWidth;
-    const int *rowSize;           // layout 0: padded to whole slices
-    const int *perm;              // layout 2: slice row -> table row
-    const int *nuniq;             // layout 2: listed control vertices per slice
-    const long long *ctrlOff;
+    const unsigned *rec;          // compact slices (stencil_compact.h), one weight array
+    const SliceDesc *slices;
+    const int *perm;              // slice row -> table row; NULL: the same
     const int *ctrl;
     const float *src;
     long long srcV, srcF;
@@ -75,14 +71,11 @@ struct BatchPatchSeg {
 // descriptors are read from memory, so the compiler would otherwise treat
 // their pointers as generic and emit flat accesses).
 #define G_ OSDHIP_GLOBAL
+#define C_ OSDHIP_CONST
 struct GStencilSeg {
     const G_ unsigned *rec;
-    const G_ long long *sliceOff;
-    const G_ int *sliceWidth;
-    const G_ int *rowSize;
+    const C_ SliceDesc *slices;
     const G_ int *perm;
-    const G_ int *nuniq;
-    const G_ long long *ctrlOff;
     const G_ int *ctrl;
     const G_ float *src;
     long long srcV, srcF;
@@ -108,17 +101,12 @@ struct GPatchSeg {
     const G_ int *ngen;
 };
 
-#define C_ OSDHIP_CONST
 __device__ __forceinline__ GStencilSeg gseg(const C_ BatchStencilSeg &s)
 {
     GStencilSeg g;
     g.rec = gptr(s.rec);
-    g.sliceOff = gptr(s.sliceOff);
-    g.sliceWidth = gptr(s.sliceWidth);
-    g.rowSize = gptr(s.rowSize);
+    g.slices = cptr(s.slices);
     g.perm = gptr(s.perm);
-    g.nuniq = gptr(s.nuniq);
-    g.ctrlOff = gptr(s.ctrlOff);
     g.ctrl = gptr(s.ctrl);
     g.src = gptr(s.src);
     g.srcV = s.srcV;
@@ -184,14 +172,6 @@ __device__ __forceinline__ osdhip_patch_param ld(const G_ osdhip_patch_param *p)
     q.field1 = p->field1;
     q.sharpness = p->sharpness;
     return q;
-}
-
-// One (index, weight) record from a global pointer (non-temporal).
-__device__ __forceinline__ void load_record_g(const OSDHIP_GLOBAL unsigned *p, int &idx, float &w)
-{
-    const v2i q = __builtin_nontemporal_load((const OSDHIP_GLOBAL v2i *)p);
-    idx = q.x;
-    w = __int_as_float(q.y);
 }
 
 struct BatchItem {
@@ -262,388 +242,284 @@ __device__ __forceinline__ int batch_next_item(const BatchArgs &a, int iter)
     return __builtin_amdgcn_readfirstlane(slot);
 }
 
-template <int LC, int FC, int G>
-__global__ __launch_bounds__(kBlock) void k_batch_stencils(BatchArgs a)
-{
-    const int lane = (int)threadIdx.x & (kWave - 1);
-    const int wv = wave_in_block();
-    for (int iter = 0;; ++iter) {
-        const int itx = batch_next_item(a, iter);
-        if (itx < 0) break;
-        const BatchItem item = ld(cptr(a.items) + itx);
-        const GStencilSeg sg = gseg(cptr(a.sseg)[item.seg]);
-        for (int sl = wv; sl < item.count; sl += kWavesPerBlock) {
-            const int s = item.first + sl;
-            const int row = s * kWave + lane;
-            const bool active = row < sg.nrows;
-            const int sz = sg.rowSize[row];
-            const int W = sg.sliceWidth[s];
-            const G_ unsigned *rp = sg.rec + (size_t)(sg.sliceOff[s] + lane) * 2;
-            for (int f0 = 0; f0 < sg.frames; f0 += FC) {
-                float acc[FC][LC];
-#pragma unroll
-                for (int c = 0; c < FC; ++c)
-#pragma unroll
-                    for (int k = 0; k < LC; ++k) acc[c][k] = 0.0f;
-                for (int j = 0; j < W; j += G) {
-                    int ii[G];
-                    float ww[1][G];
-#pragma unroll
-                    for (int u = 0; u < G; ++u)   // past the width: last column, not accumulated
-                        load_record_g(rp + (size_t)min(j + u, W - 1) * (kWave * 2), ii[u], ww[0][u]);
-                    float v[G][FC][LC];
-#pragma unroll
-                    for (int u = 0; u < G; ++u) {
-                        const G_ float *p = sg.src + (size_t)(unsigned)ii[u] * sg.srcV +
-                                                       (size_t)f0 * sg.srcF;
-#pragma unroll
-                        for (int c = 0; c < FC; ++c) {
-                            if (f0 + c < sg.frames) {           // wave-uniform
-#pragma unroll
-                                for (int k = 0; k < LC; ++k) v[u][c][k] = p[c * sg.srcF + k];
-                            } else {
-#pragma unroll
-                                for (int k = 0; k < LC; ++k) v[u][c][k] = 0.0f;
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < G; ++u) {
-                        const bool take = j + u < sz;
-#pragma unroll
-                        for (int c = 0; c < FC; ++c)
-#pragma unroll
-                            for (int k = 0; k < LC; ++k) {
-                                const float t = acc[c][k] + v[u][c][k] * ww[0][u];
-                                acc[c][k] = take ? t : acc[c][k];
-                            }
-                    }
-                }
-                if (active) {
-#pragma unroll
-                    for (int c = 0; c < FC; ++c) {
-                        if (f0 + c >= sg.frames) break;
-                        G_ float *d =
-                            sg.dst + (size_t)row * sg.dstV + (size_t)(f0 + c) * sg.dstF;
-#pragma unroll
-                        for (int k = 0; k < LC; ++k) d[k] = acc[c][k];
-                    }
-                }
-            }
-        }
-    }
-}
+// Phase A: one wave per compact slice, all frames of its segment.
+//
+// A listed slice's control vertices are staged in LDS for FC frames at a
+// time.  Each lane copies one 16-byte quad of one (vertex, frame): the lanes
+// of a load instruction cover whole vertices side by side (with the frames
+// of a vertex adjacent, 8 lines of 128 B per instruction where one vertex
+// per lane touched 64), which is what the vector cache is paid by.  The
+// quads of the next chunk are in flight, in registers, while the current
+// one is summed.
+//
+// In LDS a slot's FC * LC values lie side by side, padded (for FC > 1) to an
+// odd number of quads, so a lane reads an entry's values with 16-byte reads and slots
+// spread over all banks (109 of 128 B per clock and CU for 45 random slots
+// at FC * LC = 28, 228 B when four lanes share a slot, as neighbouring rows
+// in Far's order do; value-major 4-byte reads gave 57).
+constexpr int kBatchWidth = 16;                       // widest slice held in registers
 
-// A layout-2 slice with more distinct control vertices than LDS slots:
-// records hold control indices (padding: kTilePad, skipped); every frame in
-// turn gathers from memory and writes its results.
-template <int LC, int G>
-__device__ __forceinline__ void tiled_gather_slice(const GStencilSeg &sg, const G_ unsigned *rp, int W,
-                                                int row, bool active)
-{
-    for (int f = 0; f < sg.frames; ++f) {
-        float acc[LC];
-#pragma unroll
-        for (int k = 0; k < LC; ++k) acc[k] = 0.0f;
-        for (int j = 0; j < W; j += G) {
-            int ii[G];
-            float ww[G];
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                load_record_g(rp + (size_t)min(j + u, W - 1) * (kWave * 2), ii[u], ww[u]);
-                ii[u] = j + u < W ? ii[u] : (int)kTilePad;
-            }
-            float v[G][LC];
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                const unsigned ix = (unsigned)ii[u] == kTilePad ? 0u : (unsigned)ii[u];
-                const G_ float *p = sg.src + (size_t)ix * sg.srcV + (size_t)f * sg.srcF;
-#pragma unroll
-                for (int k = 0; k < LC; ++k) v[u][k] = p[k];
-            }
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                const bool take = (unsigned)ii[u] != kTilePad;
-#pragma unroll
-                for (int k = 0; k < LC; ++k) {
-                    const float t = acc[k] + v[u][k] * ww[u];
-                    acc[k] = take ? t : acc[k];
-                }
-            }
-        }
-        if (active) {
-            G_ float *d = sg.dst + (size_t)row * sg.dstV + (size_t)f * sg.dstF;
-#pragma unroll
-            for (int k = 0; k < LC; ++k) d[k] = acc[k];
-        }
-    }
-}
-
-// Records held in registers across every frame chunk (slices up to this
-// width: the table then leaves memory once per step).
-constexpr int kTiledRegRecords = 16;
-
-// LDS floats per wave of the layout-2 batch kernel: the staging area
-// (FC * LC values of 64 slots) doubles as the store transpose, whose rows
-// have an odd stride so that both its writes and its reads are free of bank
-// conflicts.
 template <int LC, int FC>
-struct TiledArea {
-    static constexpr int Q = FC * LC;                 // values per row and chunk
-    static constexpr int TP = Q | 1;                  // transpose row stride (odd)
-    static constexpr int SEG = Q <= 8 ? 8 : Q <= 16 ? 16 : Q <= 32 ? 32 : 64;   // lanes per row
-    static constexpr int RPI = kWave / SEG;           // rows per store instruction
-    static constexpr int FLOATS = (Q > TP ? Q : TP) * kWave;
+struct BatchChunk {
+    static constexpr int Q = FC * LC;
+    static constexpr int NQ = (Q + 3) / 4;            // quads per slot
+    // floats per slot; one frame packs its quads, so that the longest list fits
+    static constexpr int STR = FC == 1 ? 4 * NQ : 4 * (NQ | 1);
 };
+
+// Quads a lane copies per chunk (list length x quads per vertex / 64, at
+// most): lists of up to 64 vertices at FC = 4 and 5 to 8 floats, longer ones
+// at fewer frames.
+constexpr int kStageQuads = 8;
+
+// Longest list staged at FC frames: the quads a lane copies, and the LDS of
+// a wave (BatchArea).
+template <int LC, int FC, int FLOATS>
+constexpr int batch_list()
+{
+    const int byQuads = kStageQuads * kWave / (FC * ((LC + 3) / 4));
+    const int byLds = FLOATS / BatchChunk<LC, FC>::STR - 1;
+    const int n = byQuads < byLds ? byQuads : byLds;
+    return n < kSliceList ? n : kSliceList;
+}
+
+// LDS floats per wave: the longest list at one frame, 63 vertices and the
+// zero slot at FC, or the store transpose (64 rows of an odd number of
+// floats).
+template <int LC, int FC>
+struct BatchArea {
+    static constexpr int LIST = (kSliceList + 1) * BatchChunk<LC, 1>::STR;
+    static constexpr int CHUNK = kWave * BatchChunk<LC, FC>::STR;
+    static constexpr int RUNS = kWave * ((FC * LC) | 1);
+    static constexpr int MOST = LIST > CHUNK ? (LIST > RUNS ? LIST : RUNS)
+                                             : (CHUNK > RUNS ? CHUNK : RUNS);
+    static constexpr int FLOATS = (MOST + 3) / 4 * 4;
+};
+
+// The lane index through an empty asm: what a path forms from it is formed
+// there, instead of being held in registers across the whole kernel.
+__device__ __forceinline__ int lane_here()
+{
+    int lane = (int)threadIdx.x & (kWave - 1);
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
 
 // Stores a chunk's results for vertex-major outputs (dstF == LC): each lane
 // parks its row's FC * LC values in LDS, then every store instruction
 // writes RPI rows, SEG consecutive lanes per row covering the row's
 // contiguous run of FC * LC floats.
 template <int LC, int FC>
-__device__ __forceinline__ void tiled_store_runs(const GStencilSeg &sg, float *area,
-                                                 const int *rowsL, const float (&acc)[FC][LC],
-                                                 int f0)
+__device__ __forceinline__ void store_runs(const GStencilSeg &sg, float *area, const int *rowsL,
+                                           const float (&acc)[FC][LC], int f0)
 {
-    using A = TiledArea<LC, FC>;
-    const int lane = (int)threadIdx.x & (kWave - 1);
+    constexpr int Q = FC * LC, TP = Q | 1;            // odd row stride: no bank conflicts
+    constexpr int SEG = Q <= 8 ? 8 : Q <= 16 ? 16 : Q <= 32 ? 32 : 64;   // lanes per row
+    constexpr int RPI = kWave / SEG;                  // rows per store instruction
+    const int lane = lane_here();
     wave_lds_sync();                                   // compute reads of the area are done
 #pragma unroll
     for (int c = 0; c < FC; ++c)
 #pragma unroll
-        for (int k = 0; k < LC; ++k) area[lane * A::TP + c * LC + k] = acc[c][k];
+        for (int k = 0; k < LC; ++k) area[lane * TP + c * LC + k] = acc[c][k];
     wave_lds_sync();
-    const int q = lane % A::SEG, hi = lane / A::SEG;
+    const int q = lane % SEG, hi = lane / SEG;
     const int nq = min(FC, sg.frames - f0) * LC;       // valid values per row
     G_ float *base = sg.dst + (size_t)f0 * LC + q;
 #pragma unroll 4
-    for (int it = 0; it < kWave / A::RPI; ++it) {
-        const int r = it * A::RPI + hi;
+    for (int it = 0; it < kWave / RPI; ++it) {
+        const int r = it * RPI + hi;
         const int rr = rowsL[r];
-        if (q < nq && rr >= 0) base[(size_t)rr * sg.dstV] = area[r * A::TP + q];
+        if (q < nq && rr >= 0) base[(size_t)rr * sg.dstV] = area[r * TP + q];
     }
 }
 
-// One listed layout-2 slice for every frame, FC frames per chunk: the
-// wave stages its listed control vertices' frames into LDS (lane u ->
-// slot u), then accumulates each row's entries from LDS.  RES: the slice's
-// (up to N) records are loaded once into registers; otherwise they are read
-// N per group for every chunk.
-template <int LC, int FC, int N, bool RES, int G>
-__device__ __forceinline__ void tiled_lds_slice(const GStencilSeg &sg, float *area, int *rowsL,
-                                                const G_ unsigned *rp, int W, int U, int vtx,
-                                                int row, bool active)
+// acc[c][k] += the first NF * LC values at p times w.
+template <int LC, int FC, int NF>
+__device__ __forceinline__ void add_entry(const float *p, float w, float (&acc)[FC][LC])
 {
-    const int lane = (int)threadIdx.x & (kWave - 1);
-    float(*Ls)[kTileSlots] = (float(*)[kTileSlots])area;
+    constexpr int NQ = (NF * LC + 3) / 4;
+    float x[4 * NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const v4f v = *(const v4f *)(p + 4 * q);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[4 * q + k] = v[k];
+    }
+#pragma unroll
+    for (int c = 0; c < NF; ++c)
+#pragma unroll
+        for (int k = 0; k < LC; ++k) acc[c][k] = acc[c][k] + x[c * LC + k] * w;
+}
+
+// One listed slice for every frame, FC per chunk (U <= batch_list at FC).
+// RES: the slice's entries (W <= kBatchWidth) stay in registers.
+template <int LC, int FC, bool RES>
+__device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float *area, int *rowsL,
+                                                   const G_ unsigned *rp, const G_ float *wp, int W,
+                                                   int U, const G_ int *list, int row, bool active)
+{
+    using A = BatchChunk<LC, FC>;
+    constexpr int GR = RES ? kBatchWidth / 4 : 1;      // entry groups held
+    constexpr int H = (LC + 3) / 4;                    // quads per (vertex, frame)
+    constexpr int N = LC < 4 ? LC : 4;                 // floats per copied quad
+    constexpr int QV = FC * H;                         // quads per vertex: 1, 2, 4 or 8
+    constexpr int VI = kWave / QV;                     // vertices per copy instruction
+    constexpr int LISTS = (kStageQuads + QV - 1) / QV; // list registers (64 vertices each)
+    const int lane = lane_here();
+    const int G = (W + 3) / 4;
+    EntryGroup<1> e[GR];
+    auto load = [&](int g0) {
+#pragma unroll
+        for (int c = 0; c < GR; ++c)
+            if (g0 + c < G) {                          // wave-uniform
+                e[c].slots = __builtin_nontemporal_load(rp + (size_t)(g0 + c) * kWave + lane);
+                load_weights<1>(wp, W, g0 + c, lane, e[c].w);
+            }
+    };
+    int vtx[LISTS];
+#pragma unroll
+    for (int h = 0; h < LISTS; ++h) {
+        vtx[h] = 0;
+        if (h * kWave < U) vtx[h] = list[min(h * kWave + lane, U - 1)];
+    }
+    if (RES) load(0);
+    // this lane's quad of its vertices: frame c of the chunk, floats
+    // [k0, k0 + N) (the last quad of 5 to 7 floats overlaps the one before)
+    const int q = lane % QV, c = q / H, k0 = min(4 * (q % H), LC - N);
+    float x[kStageQuads][N];
+    auto stage = [&](int f0) {
+        // frames past the end repeat the last one (never stored)
+        const G_ float *p = sg.src + (size_t)min(f0 + c, sg.frames - 1) * sg.srcF + k0;
+#pragma unroll
+        for (int r = 0; r < kStageQuads; ++r)
+            if (r * VI < U) {                          // wave-uniform
+                const int v = __shfl(vtx[r / QV], (r * VI + lane / QV) % kWave, kWave);
+                const G_ float *pv = p + (size_t)(unsigned)v * sg.srcV;
+#pragma unroll
+                for (int k = 0; k < N; ++k) x[r][k] = pv[k];
+            }
+    };
     // vertex-major outputs with a row's frames adjacent: results leave
-    // through LDS so that consecutive lanes store one row's run (measured
-    // faster than per-lane stores for that layout; frame-major outputs keep
-    // per-lane stores, which are faster still)
+    // through LDS so that consecutive lanes store one row's run
     const bool runs = sg.dstF == LC && sg.frames > 1;
     if (runs) rowsL[lane] = active ? row : -1;
-    int slot[N];
-    float ww[N];
-    auto load = [&](int j0) {
-#pragma unroll
-        for (int u = 0; u < N; ++u) {
-            // unconditional loads; past the width: the zero slot
-            load_record_g(rp + (size_t)min(j0 + u, W - 1) * (kWave * 2), slot[u], ww[u]);
-            slot[u] = j0 + u < W ? slot[u] : kTileZero;
-            ww[u] = j0 + u < W ? ww[u] : 0.0f;
-        }
-    };
-    if (RES) load(0);
+    stage(0);
     for (int f0 = 0; f0 < sg.frames; f0 += FC) {
+        wave_lds_sync();                               // previous chunk's reads are done
+#pragma unroll
+        for (int r = 0; r < kStageQuads; ++r) {
+            const int u = r * VI + lane / QV;
+            if (r * VI < U && u < U) {
+                float *d = area + u * A::STR + c * LC + k0;
+#pragma unroll
+                for (int k = 0; k < N; ++k) d[k] = x[r][k];
+            }
+        }
+        if (lane < A::STR) area[U * A::STR + lane] = 0.0f;   // the zero slot
+        wave_lds_sync();
+        // the next chunk's loads are in flight while this one is summed
+        if (f0 + FC < sg.frames) stage(f0 + FC);
         float acc[FC][LC];
 #pragma unroll
-        for (int c = 0; c < FC; ++c)
+        for (int f = 0; f < FC; ++f)
 #pragma unroll
-            for (int k = 0; k < LC; ++k) acc[c][k] = 0.0f;
-        wave_lds_sync();                                 // previous chunk's reads are done
-        if (lane < U) {
-            const G_ float *p = sg.src + (size_t)(unsigned)vtx * sg.srcV + (size_t)f0 * sg.srcF;
+            for (int k = 0; k < LC; ++k) acc[f][k] = 0.0f;
+        auto entries = [&](auto frames) {
+            constexpr int NF = decltype(frames)::value;
+            for (int g0 = 0; g0 < (RES ? 1 : G); g0 += GR) {
+                if (!RES) load(g0);
 #pragma unroll
-            for (int c = 0; c < FC; ++c) {
-                if (f0 + c < sg.frames) {                   // wave-uniform
+                for (int g = 0; g < GR; ++g) {
+                    if (g0 + g < G) {                  // wave-uniform
+                        // through an empty asm each chunk: the LDS addresses
+                        // are formed per chunk instead of held across the
+                        // frame loop
+                        unsigned slots = e[g].slots;
+                        asm volatile("" : "+v"(slots));
 #pragma unroll
-                    for (int k = 0; k < LC; ++k) Ls[c * LC + k][lane] = p[c * sg.srcF + k];
-                }
-            }
-        } else if (lane == kTileZero) {                  // the store transpose reuses the area
-#pragma unroll
-            for (int q = 0; q < FC * LC; ++q) Ls[q][kTileZero] = 0.0f;
-        }
-        wave_lds_sync();
-        for (int j0 = 0; j0 < (RES ? 1 : W); j0 += N) {
-            if (!RES) load(j0);
-#pragma unroll
-            for (int u = 0; u < N; ++u) {
-                if (RES && u >= W) break;                   // wave-uniform
-#pragma unroll
-                for (int c = 0; c < FC; ++c)
-#pragma unroll
-                    for (int k = 0; k < LC; ++k)
-                        acc[c][k] = acc[c][k] + Ls[c * LC + k][slot[u]] * ww[u];
-                // one entry's LDS reads in flight at a time: hoisting all
-                // of them would cut occupancy
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        if (runs) {
-            tiled_store_runs<LC, FC>(sg, area, rowsL, acc, f0);
-        } else if (active) {
-#pragma unroll
-            for (int c = 0; c < FC; ++c) {
-                if (f0 + c >= sg.frames) break;
-                G_ float *d = sg.dst + (size_t)row * sg.dstV + (size_t)(f0 + c) * sg.dstF;
-#pragma unroll
-                for (int k = 0; k < LC; ++k) d[k] = acc[c][k];
-            }
-        }
-    }
-}
-
-// Phase A on locality-ordered tables (layout 2): per slice and chunk of FC
-// frames, the wave stages the slice's listed control vertices (one per
-// lane, FC frames each) into its LDS region, element (c, k) of slot u at
-// lds[c * LC + k][u], then accumulates every entry from LDS; a slice's
-// records stay in registers for all its chunks (slices of width up to
-// kTiledRegRecords) or are re-read per chunk.  Results go to the table row
-// perm[slice row].  Unlisted slices gather from memory.
-template <int LC, int FC, int G>
-__global__ __launch_bounds__(kBlock) void k_batch_stencils_tiled(BatchArgs a)
-{
-    __shared__ float lds[kWavesPerBlock][TiledArea<LC, FC>::FLOATS];
-    __shared__ int rowsLds[kWavesPerBlock][kWave];
-    const int lane = (int)threadIdx.x & (kWave - 1);
-    const int wv = wave_in_block();
-    for (int iter = 0;; ++iter) {
-        const int itx = batch_next_item(a, iter);
-        if (itx < 0) break;
-        const BatchItem item = ld(cptr(a.items) + itx);
-        const GStencilSeg sg = gseg(cptr(a.sseg)[item.seg]);
-        for (int sl = wv; sl < item.count; sl += kWavesPerBlock) {
-            const int s = item.first + sl;
-            const int row = sg.perm[(long long)s * kWave + lane];
-            const bool active = row < sg.nrows;
-            const int W = sg.sliceWidth[s];
-            const int U = sg.nuniq[s];
-            const G_ unsigned *rp = sg.rec + (size_t)(sg.sliceOff[s] + lane) * 2;
-            if (U < 0) {
-                // rare: more distinct control vertices than LDS slots; one
-                // frame at a time, gathers from memory
-                tiled_gather_slice<LC, G>(sg, rp, W, row, active);
-                continue;
-            }
-            const int vtx = lane < U ? sg.ctrl[sg.ctrlOff[s] + lane] : 0;
-            if (W <= kTiledRegRecords)
-                tiled_lds_slice<LC, FC, kTiledRegRecords, true, G>(sg, lds[wv], rowsLds[wv], rp, W,
-                                                                   U, vtx, row, active);
-            else
-                tiled_lds_slice<LC, FC, G, false, G>(sg, lds[wv], rowsLds[wv], rp, W, U, vtx, row,
-                                                     active);
-        }
-    }
-}
-
-// Phase A with the slice's records held in registers for all frames: a
-// slice of width W <= 16 loads its (index, weight) records once, then every
-// frame gathers and accumulates from registers, so the table leaves HBM
-// exactly once per step whatever the frame count.  Wider slices take the
-// chunked path (one frame per chunk, gather group 4).
-template <int LC>
-__global__ __launch_bounds__(kBlock) void k_batch_stencils_rr(BatchArgs a)
-{
-    constexpr int MAXW = 16, GG = 4;
-    const int lane = (int)threadIdx.x & (kWave - 1);
-    const int wv = wave_in_block();
-    for (int iter = 0;; ++iter) {
-        const int itx = batch_next_item(a, iter);
-        if (itx < 0) break;
-        const BatchItem item = ld(cptr(a.items) + itx);
-        const GStencilSeg sg = gseg(cptr(a.sseg)[item.seg]);
-        for (int sl = wv; sl < item.count; sl += kWavesPerBlock) {
-            const int s = item.first + sl;
-            const int row = s * kWave + lane;
-            const bool active = row < sg.nrows;
-            const int sz = sg.rowSize[row];
-            const int W = sg.sliceWidth[s];
-            const G_ unsigned *rp = sg.rec + (size_t)(sg.sliceOff[s] + lane) * 2;
-            if (W <= MAXW) {
-                int ii[MAXW];
-                float ww[1][MAXW];
-#pragma unroll
-                for (int j = 0; j < MAXW; ++j)    // past the width: last column, not accumulated
-                    load_record_g(rp + (size_t)min(j, W - 1) * (kWave * 2), ii[j], ww[0][j]);
-                for (int f = 0; f < sg.frames; ++f) {
-                    float acc[LC];
-#pragma unroll
-                    for (int k = 0; k < LC; ++k) acc[k] = 0.0f;
-                    const G_ float *base = sg.src + (size_t)f * sg.srcF;
-#pragma unroll
-                    for (int j0 = 0; j0 < MAXW; j0 += GG) {
-                        if (j0 < W) {                            // wave-uniform
-                            float v[GG][LC];
-#pragma unroll
-                            for (int u = 0; u < GG; ++u) {
-                                const G_ float *p = base + (size_t)(unsigned)ii[j0 + u] * sg.srcV;
-#pragma unroll
-                                for (int k = 0; k < LC; ++k) v[u][k] = p[k];
-                            }
-#pragma unroll
-                            for (int u = 0; u < GG; ++u) {
-                                const bool take = j0 + u < sz;
-#pragma unroll
-                                for (int k = 0; k < LC; ++k) {
-                                    const float t = acc[k] + v[u][k] * ww[0][j0 + u];
-                                    acc[k] = take ? t : acc[k];
-                                }
-                            }
+                        for (int u = 0; u < 4; ++u) {
+                            add_entry<LC, FC, NF>(area + ((slots >> (8 * u)) & 0xffu) * A::STR,
+                                                  e[g].w[0][u], acc);
+                            // one entry's LDS reads in flight at a time:
+                            // hoisting all of them would cut occupancy
+                            __builtin_amdgcn_sched_barrier(0);
                         }
                     }
+                }
+            }
+        };
+        // a last chunk of at most half its frames reads and adds only those
+        if (FC > 1 && sg.frames - f0 <= FC / 2)        // wave-uniform
+            entries(std::integral_constant<int, (FC + 1) / 2>{});
+        else
+            entries(std::integral_constant<int, FC>{});
+        if (runs) {
+            store_runs<LC, FC>(sg, area, rowsL, acc, f0);
+        } else if (active) {
+#pragma unroll
+            for (int f = 0; f < FC; ++f) {
+                if (f0 + f >= sg.frames) break;
+                G_ float *d = sg.dst + (size_t)row * sg.dstV + (size_t)(f0 + f) * sg.dstF;
+#pragma unroll
+                for (int k = 0; k < LC; ++k) d[k] = acc[f][k];
+            }
+        }
+    }
+}
+
+template <int LC, int FC>
+__global__ __launch_bounds__(kBlock) void k_batch_stencils(BatchArgs a)
+{
+    constexpr int FLOATS = BatchArea<LC, FC>::FLOATS;
+    __shared__ __attribute__((aligned(16))) float lds[kWavesPerBlock][FLOATS];
+    __shared__ int rowsLds[kWavesPerBlock][kWave];
+    const int wv = wave_in_block();
+    for (int iter = 0;; ++iter) {
+        const int itx = batch_next_item(a, iter);
+        if (itx < 0) break;
+        const BatchItem item = ld(cptr(a.items) + itx);
+        const GStencilSeg sg = gseg(cptr(a.sseg)[item.seg]);
+        for (int sl = wv; sl < item.count; sl += kWavesPerBlock) {
+            const int s = item.first + sl, lane = lane_here();
+            const C_ SliceDesc &ds = sg.slices[s];     // scalar loads
+            const int W = ds.width, U = ds.nuniq;
+            int row = s * kWave + lane;
+            if (sg.perm) row = sg.perm[(long long)s * kWave + lane];
+            const bool active = row < sg.nrows;
+            const G_ unsigned *rp = sg.rec + ds.off;
+            const G_ float *wp = (const G_ float *)(rp + slice_index_dwords(W, U));
+            if (U < 0) {
+                // more distinct control vertices than a list holds: one
+                // frame at a time, gathers from memory
+                for (int f = 0; f < sg.frames; ++f) {
+                    float acc[1][LC];
+#pragma unroll
+                    for (int k = 0; k < LC; ++k) acc[0][k] = 0.0f;
+                    gather_slice<1, LC>(sg.src + (size_t)f * sg.srcF, (size_t)sg.srcV, rp, wp, W,
+                                        lane, acc);
                     if (active) {
                         G_ float *d = sg.dst + (size_t)row * sg.dstV + (size_t)f * sg.dstF;
 #pragma unroll
-                        for (int k = 0; k < LC; ++k) d[k] = acc[k];
+                        for (int k = 0; k < LC; ++k) d[k] = acc[0][k];
                     }
                 }
                 continue;
             }
-            for (int f = 0; f < sg.frames; ++f) {
-                float acc[LC];
-#pragma unroll
-                for (int k = 0; k < LC; ++k) acc[k] = 0.0f;
-                for (int j = 0; j < W; j += GG) {
-                    int ii[GG];
-                    float ww[1][GG];
-#pragma unroll
-                    for (int u = 0; u < GG; ++u)
-                        load_record_g(rp + (size_t)min(j + u, W - 1) * (kWave * 2), ii[u], ww[0][u]);
-                    float v[GG][LC];
-#pragma unroll
-                    for (int u = 0; u < GG; ++u) {
-                        const G_ float *p = sg.src + (size_t)(unsigned)ii[u] * sg.srcV +
-                                         (size_t)f * sg.srcF;
-#pragma unroll
-                        for (int k = 0; k < LC; ++k) v[u][k] = p[k];
-                    }
-#pragma unroll
-                    for (int u = 0; u < GG; ++u) {
-                        const bool take = j + u < sz;
-#pragma unroll
-                        for (int k = 0; k < LC; ++k) {
-                            const float t = acc[k] + v[u][k] * ww[0][u];
-                            acc[k] = take ? t : acc[k];
-                        }
-                    }
-                }
-                if (active) {
-                    G_ float *d = sg.dst + (size_t)row * sg.dstV + (size_t)f * sg.dstF;
-#pragma unroll
-                    for (int k = 0; k < LC; ++k) d[k] = acc[k];
-                }
-            }
+            const G_ int *list = sg.ctrl + ds.ctrlOff;
+            float *area = lds[wv];
+            int *rowsL = rowsLds[wv];
+            // a list too long for FC frames at once takes fewer per chunk
+            static_assert(batch_list<LC, 1, FLOATS>() == kSliceList, "every list fits at one frame");
+            if (W > kBatchWidth)
+                batch_listed_slice<LC, 1, false>(sg, area, rowsL, rp, wp, W, U, list, row, active);
+            else if (FC == 4 && U <= batch_list<LC, FC, FLOATS>())
+                batch_listed_slice<LC, FC, true>(sg, area, rowsL, rp, wp, W, U, list, row, active);
+            else if (FC >= 2 && U <= batch_list<LC, FC < 2 ? 1 : 2, FLOATS>())
+                batch_listed_slice<LC, FC < 2 ? 1 : 2, true>(sg, area, rowsL, rp, wp, W, U, list,
+                                                             row, active);
+            else
+                batch_listed_slice<LC, 1, true>(sg, area, rowsL, rp, wp, W, U, list, row, active);
         }
     }
 }

@@ -31,36 +31,13 @@
 #include "patch_map.h"
 #include "tess.h"
 #include "patch_sort.h"
+#include "stencil_compact.h"
 #include "stencil_csr.h"
 #include "stencil_sliced.h"
-#include "stencil_tiled.h"
 #include "table.h"
 #include "table_build.h"
 
 namespace osdhip {
-
-template <int NWT, int G>
-static void launch_rec_g(int lc, const RecArgs &a, int grid, hipStream_t st)
-{
-    switch (lc) {
-    case 1: hipLaunchKernelGGL((k_stencils_rec<NWT, 1, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((k_stencils_rec<NWT, 2, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 3: hipLaunchKernelGGL((k_stencils_rec<NWT, 3, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((k_stencils_rec<NWT, 4, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 5: hipLaunchKernelGGL((k_stencils_rec<NWT, 5, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 6: hipLaunchKernelGGL((k_stencils_rec<NWT, 6, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 7: hipLaunchKernelGGL((k_stencils_rec<NWT, 7, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    default: hipLaunchKernelGGL((k_stencils_rec<NWT, 8, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    }
-}
-
-template <int NWT>
-static void launch_rec(int lc, int group, const RecArgs &a, int grid, hipStream_t st)
-{
-    if (group == 4) launch_rec_g<NWT, 4>(lc, a, grid, st);
-    else if (group == 16) launch_rec_g<NWT, 16>(lc, a, grid, st);
-    else launch_rec_g<NWT, 8>(lc, a, grid, st);
-}
 
 template <int G>
 static void launch_rec_paired_g(int lc, const RecArgs &a, int grid, hipStream_t st)
@@ -84,26 +61,23 @@ static void launch_rec_paired(int lc, int group, const RecArgs &a, int grid, hip
     else launch_rec_paired_g<8>(lc, a, grid, st);
 }
 
-template <int NWT, int G>
-static void launch_tiled_g(int lc, const TiledArgs &a, int grid, hipStream_t st)
-{
-    switch (lc) {
-    case 1: hipLaunchKernelGGL((k_stencils_tiled<NWT, 1, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((k_stencils_tiled<NWT, 2, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 3: hipLaunchKernelGGL((k_stencils_tiled<NWT, 3, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((k_stencils_tiled<NWT, 4, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 5: hipLaunchKernelGGL((k_stencils_tiled<NWT, 5, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 6: hipLaunchKernelGGL((k_stencils_tiled<NWT, 6, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 7: hipLaunchKernelGGL((k_stencils_tiled<NWT, 7, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    default: hipLaunchKernelGGL((k_stencils_tiled<NWT, 8, G>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    }
-}
-
 template <int NWT>
-static void launch_tiled(int lc, int group, const TiledArgs &a, int grid, hipStream_t st)
+static void launch_compact(int lc, const CompactArgs &a, int grid, hipStream_t st)
 {
-    if (group == 4) launch_tiled_g<NWT, 4>(lc, a, grid, st);
-    else launch_tiled_g<NWT, 8>(lc, a, grid, st);
+    // dynamic LDS: four waves' slots (at most 4 * 256 * 32 B)
+    const size_t lds = sizeof(float) * kWavesPerBlock * (size_t)a.slots *
+                       (lc == 1 ? SlotShape<1>::STR : lc == 2 ? SlotShape<2>::STR
+                                : lc <= 4 ? SlotShape<4>::STR : SlotShape<8>::STR);
+    switch (lc) {
+    case 1: hipLaunchKernelGGL((k_stencils_compact<NWT, 1>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    case 2: hipLaunchKernelGGL((k_stencils_compact<NWT, 2>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    case 3: hipLaunchKernelGGL((k_stencils_compact<NWT, 3>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    case 4: hipLaunchKernelGGL((k_stencils_compact<NWT, 4>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    case 5: hipLaunchKernelGGL((k_stencils_compact<NWT, 5>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    case 6: hipLaunchKernelGGL((k_stencils_compact<NWT, 6>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    case 7: hipLaunchKernelGGL((k_stencils_compact<NWT, 7>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    default: hipLaunchKernelGGL((k_stencils_compact<NWT, 8>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    }
 }
 
 template <int NW, bool VEC>
@@ -230,9 +204,9 @@ static void free_table(osdhip_stencil_table *t)
 {
     if (!t) return;
     void *ptrs[] = { t->sizes, t->offsets, t->indices, t->w[0], t->w[1], t->w[2], t->w[3],
-                     t->w[4], t->w[5], t->sliceOff, t->sliceWidth, t->rowSize, t->rec, t->sidx,
-                     t->sw[0], t->sw[1], t->sw[2], t->sw[3], t->sw[4], t->sw[5], t->perm,
-                     t->nuniq, t->ctrlOff, t->ctrl };
+                     t->w[4], t->w[5], t->slices, t->perm, t->ctrl, t->rec, t->sliceOff,
+                     t->sliceWidth, t->rowSize, t->sidx, t->sw[0], t->sw[1], t->sw[2], t->sw[3],
+                     t->sw[4], t->sw[5] };
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete t;
@@ -258,130 +232,149 @@ static bool upload(T **dptr, const T *host, size_t count, hipStream_t st, long l
     return hipMemcpyAsync(*dptr, host, count * sizeof(T), hipMemcpyHostToDevice, st) == hipSuccess;
 }
 
-// Exclusive prefix sum of n counts into out; returns the total (-1 on error).
-template <typename T>
-static long long exclusive_scan(const T *counts, T *out, int n, hipStream_t st)
-{
-    size_t bytes = 0;
-    void *tmp = nullptr;
-    if (hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, counts, out, n, st) != hipSuccess ||
-        hipMalloc(&tmp, std::max<size_t>(bytes, 1)) != hipSuccess)
-        return -1;
-    T last[2] = { 0, 0 };
-    const bool ok =
-        hipcub::DeviceScan::ExclusiveSum(tmp, bytes, counts, out, n, st) == hipSuccess &&
-        hipMemcpyAsync(&last[0], out + (n - 1), sizeof(T), hipMemcpyDeviceToHost, st) == hipSuccess &&
-        hipMemcpyAsync(&last[1], counts + (n - 1), sizeof(T), hipMemcpyDeviceToHost, st) ==
-            hipSuccess &&
-        hipStreamSynchronize(st) == hipSuccess;
-    (void)hipFree(tmp);
-    return ok ? (long long)last[0] + (long long)last[1] : -1;
-}
+// Tables of fewer rows keep the dominant order under order 2.
+constexpr int kFarOrderRows = 1 << 16;
 
-// Layout 2 from the uploaded CSR arrays: dominant-vertex row order (stable
-// radix sort), optionally regrouped by row size within windows of 128 or 512
-// rows, per-slice widths and control lists (count pass, scans, fill pass).
-static bool build_tiled(osdhip_stencil_table *t, hipStream_t st)
+// Compact slices (layouts 0 and 2) from the uploaded CSR arrays: the row
+// order (Far's; or by dominant vertex, a stable radix sort, optionally
+// regrouped by row size within windows of 128 or 512 rows), then per-slice
+// widths and control lists (count pass, scan, fill pass).
+static bool build_compact(osdhip_stencil_table *t, hipStream_t st)
 {
     const int n = t->n, S = t->nslices, rows = S * kWave;
-    long long scratchBytes = 0;
-    unsigned *keys = nullptr, *keysOut = nullptr;
-    int *vals = nullptr;
-    long long *entries = nullptr, *listLen = nullptr;
-    void *sortTmp = nullptr;
-    size_t sortBytes = 0;
+    bool farOrder = t->layout == 0 || t->order == 1;
+    const bool maySort = !farOrder;
+    int cap = farOrder ? kSliceList : kLocalityList;
+    const SliceCount zero = { 0, 0, 0, 0, 0 };
+    size_t scanBytes = 0, sortBytes = 0;
+    if (hipcub::DeviceScan::ExclusiveScan(nullptr, scanBytes, (SliceCount *)nullptr,
+                                          (SliceCount *)nullptr, SliceCountAdd(), zero, S, st) !=
+            hipSuccess ||
+        (maySort && hipcub::DeviceRadixSort::SortPairs(nullptr, sortBytes, (unsigned *)nullptr,
+                                                       (unsigned *)nullptr, (int *)nullptr,
+                                                       (int *)nullptr, rows, 0, 32, st) != hipSuccess))
+        return false;
+    // one scratch allocation for every array the build needs
+    size_t used = 0;
+    auto part = [&](size_t bytes) {
+        const size_t at = used;
+        used += (bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    const size_t oCounts = part(sizeof(SliceCount) * S), oBefore = part(sizeof(SliceCount) * S),
+                 oWidth = part(sizeof(int) * S), oUniq = part(sizeof(int) * S),
+                 oTmp = part(std::max(scanBytes, sortBytes)),
+                 oKeys = part(maySort ? sizeof(int) * (size_t)rows : 0),
+                 oKeep = part(maySort ? sizeof(int) * (size_t)rows : 0),
+                 oVals = part(maySort ? sizeof(int) * (size_t)rows : 0);
+    char *scratch = nullptr;
+    if (hipMalloc((void **)&scratch, used) != hipSuccess) return false;
+    SliceCount *counts = (SliceCount *)(scratch + oCounts), *before = (SliceCount *)(scratch + oBefore);
+    int *width = (int *)(scratch + oWidth), *nuniq = (int *)(scratch + oUniq);
+    unsigned *keys = (unsigned *)(scratch + oKeys);
+    int *keep = (int *)(scratch + oKeep), *vals = (int *)(scratch + oVals);
+    void *tmp = scratch + oTmp;
     const int gr = (rows + kBlock - 1) / kBlock, gs = (S + kWavesPerBlock - 1) / kWavesPerBlock;
     const float *const *W = t->w;
-    bool ok = dalloc(&keys, (size_t)rows, scratchBytes) && dalloc(&keysOut, (size_t)rows, scratchBytes) &&
-              dalloc(&vals, (size_t)rows, scratchBytes) && dalloc(&entries, (size_t)S, scratchBytes) &&
-              dalloc(&listLen, (size_t)S, scratchBytes) && dalloc(&t->perm, (size_t)rows, t->bytes) &&
-              dalloc(&t->sliceWidth, (size_t)S, t->bytes) && dalloc(&t->sliceOff, (size_t)S, t->bytes) &&
-              dalloc(&t->nuniq, (size_t)S, t->bytes) && dalloc(&t->ctrlOff, (size_t)S, t->bytes);
-    if (ok) {
-        hipLaunchKernelGGL(k_row_dominant, dim3(gr), dim3(kBlock), 0, st, t->sizes, t->offsets,
-                           t->indices, W[0], n, rows, t->order == 1 ? 1 : 0, keys, vals);
-        ok = hipcub::DeviceRadixSort::SortPairs(nullptr, sortBytes, keys, keysOut, vals, t->perm, rows,
-                                                0, 32, st) == hipSuccess &&
-             hipMalloc(&sortTmp, std::max<size_t>(sortBytes, 1)) == hipSuccess &&
-             hipcub::DeviceRadixSort::SortPairs(sortTmp, sortBytes, keys, keysOut, vals, t->perm,
-                                                rows, 0, 32, st) == hipSuccess;
-    }
-#define OSDHIP_TILED(NWT, FILL, PERM)                                                           \
-    hipLaunchKernelGGL((k_tiled_slices<NWT, FILL>), dim3(gs), dim3(kBlock), 0, st, PERM,        \
-                       t->sizes, t->offsets, t->indices, W[0], W[1], W[2], W[3], W[4], W[5], n, \
-                       S, t->sliceWidth, entries, t->nuniq, listLen, t->sliceOff, t->ctrlOff,   \
-                       t->ctrl, t->rec)
-    // count pass over a row order: slice widths and entries, control-list
-    // counts; `listed` receives the slices that list their control vertices
-    auto countPass = [&](const int *perm, int &listed) -> bool {
-        if (t->nw == 1) OSDHIP_TILED(1, false, perm);
-        else if (t->nw == 3) OSDHIP_TILED(3, false, perm);
-        else OSDHIP_TILED(6, false, perm);
-        std::unique_ptr<int[]> nu(new (std::nothrow) int[(size_t)S]);
-        const bool good = hipGetLastError() == hipSuccess && nu &&
-                          hipMemcpyAsync(nu.get(), t->nuniq, (size_t)S * sizeof(int),
-                                         hipMemcpyDeviceToHost, st) == hipSuccess &&
-                          hipStreamSynchronize(st) == hipSuccess;
-        if (good)
-            listed = (int)std::count_if(nu.get(), nu.get() + S, [](int u) { return u >= 0; });
+    bool ok = dalloc(&t->slices, (size_t)S, t->bytes);
+#define OSDHIP_COMPACT(NWT, FILL, PERM)                                                          \
+    hipLaunchKernelGGL((k_compact_slices<NWT, FILL>), dim3(gs), dim3(kBlock), 0, st, PERM,       \
+                       t->sizes, t->offsets, t->indices, W[0], W[1], W[2], W[3], W[4], W[5], n,  \
+                       S, cap, width, nuniq, counts, before, t->slices, t->ctrl, t->rec)
+    // count pass and scan over a row order; the totals over all slices
+    auto count = [&](const int *perm, SliceCount &total) -> bool {
+        if (t->nw == 1) OSDHIP_COMPACT(1, false, perm);
+        else if (t->nw == 3) OSDHIP_COMPACT(3, false, perm);
+        else OSDHIP_COMPACT(6, false, perm);
+        SliceCount last[2];
+        size_t bytes = scanBytes;
+        const bool good =
+            hipGetLastError() == hipSuccess &&
+            hipcub::DeviceScan::ExclusiveScan(tmp, bytes, counts, before, SliceCountAdd(), zero, S,
+                                              st) == hipSuccess &&
+            hipMemcpyAsync(&last[0], before + (S - 1), sizeof(SliceCount), hipMemcpyDeviceToHost,
+                           st) == hipSuccess &&
+            hipMemcpyAsync(&last[1], counts + (S - 1), sizeof(SliceCount), hipMemcpyDeviceToHost,
+                           st) == hipSuccess &&
+            hipStreamSynchronize(st) == hipSuccess;
+        if (good) total = SliceCountAdd()(last[0], last[1]);
         return good;
     };
-    int listed = 0;
-    if (ok) ok = countPass(t->perm, listed);
-    // Size windows (order 0): of the dominant order
-    // and its regroupings by size within 128- and 512-row windows, keep the
-    // one whose slices hold the fewest record entries among those that list
-    // as many slices as the dominant order.  The winner is kept in keysOut
-    // (free after the sort), candidates are built in vals.
+    SliceCount total = zero;
+    if (ok && farOrder) ok = count(nullptr, total);
+    // Order 2 (many-frame batches) keeps Far's order where its slices list
+    // few control vertices.  A batch writes each frame's rows to a region of
+    // its own, past what the caches hold, and the dominant order's scattered
+    // 28-byte rows then bound it: a level-4 table of 4.0 M rows, 14 frames of
+    // 7 floats, takes 0.78 ms in the dominant order (writes alone 0.65 ms)
+    // and 0.66 ms in Far's (0.40 ms), with 0.46 list entries per row; level 3
+    // (0.84 per row) takes 0.084 against 0.096 ms, level 2 (1.6) 0.065
+    // against 0.14 ms.  Below kFarOrderRows rows the outputs stay in the
+    // caches and the dominant order is kept.
+    if (ok && !farOrder && t->order == 2 && n >= kFarOrderRows) {
+        cap = kSliceList;
+        ok = count(nullptr, total);
+        farOrder = total.listed >= S - S / 256 && 2 * total.list <= n;
+        if (!farOrder) cap = kLocalityList;
+    }
     t->sizeWindow = 0;
-    if (ok && t->order == 0 && S > 1) {
-        long long best = exclusive_scan(entries, t->sliceOff, S, st);
-        ok = best >= 0;
-        int *cand = vals, *keep = (int *)keysOut;
-        const int base = listed;
-        for (int K : { 128, 512 }) {
-            if (!ok) break;
-            const long long nwin = ((long long)rows + K - 1) / K;
-            if (K == 128)
-                hipLaunchKernelGGL(k_window_size_sort<128>, dim3((unsigned)nwin), dim3(kBlock), 0, st,
-                                   t->perm, t->sizes, n, (long long)rows, cand);
-            else
-                hipLaunchKernelGGL(k_window_size_sort<512>, dim3((unsigned)nwin), dim3(kBlock), 0, st,
-                                   t->perm, t->sizes, n, (long long)rows, cand);
-            int l = 0;
-            ok = hipGetLastError() == hipSuccess && countPass(cand, l);
-            const long long e = ok ? exclusive_scan(entries, t->sliceOff, S, st) : -1;
-            ok = ok && e >= 0;
-            if (ok && l >= base && e < best) {
-                best = e;
-                t->sizeWindow = K;
-                ok = hipMemcpyAsync(keep, cand, (size_t)rows * sizeof(int), hipMemcpyDeviceToDevice,
-                                    st) == hipSuccess;
-            }
+    if (ok && !farOrder) {
+        ok = dalloc(&t->perm, (size_t)rows, t->bytes);
+        if (ok) {
+            size_t bytes = sortBytes;
+            hipLaunchKernelGGL(k_row_dominant, dim3(gr), dim3(kBlock), 0, st, t->sizes, t->offsets,
+                               t->indices, W[0], n, rows, keys, vals);
+            ok = hipcub::DeviceRadixSort::SortPairs(tmp, bytes, keys, (unsigned *)keep, vals, t->perm,
+                                                    rows, 0, 32, st) == hipSuccess &&
+                 count(t->perm, total);
         }
-        if (ok && t->sizeWindow)
-            ok = hipMemcpyAsync(t->perm, keep, (size_t)rows * sizeof(int), hipMemcpyDeviceToDevice,
-                                st) == hipSuccess;
-        if (ok) ok = countPass(t->perm, listed);      // the counts of the kept order
+        // Size windows (order 0): of the dominant order and its regroupings
+        // by size within 128- and 512-row windows, keep the one whose slices
+        // hold the fewest entries among those that list as many slices as
+        // the dominant order.  The winner is kept in `keep` (free after the
+        // sort), candidates are built in vals.
+        if (ok && t->order == 0 && S > 1) {
+            const int base = total.listed;
+            SliceCount best = total;
+            for (int K : { 128, 512 }) {
+                if (!ok) break;
+                const long long nwin = ((long long)rows + K - 1) / K;
+                if (K == 128)
+                    hipLaunchKernelGGL(k_window_size_sort<128>, dim3((unsigned)nwin), dim3(kBlock), 0,
+                                       st, t->perm, t->sizes, n, (long long)rows, vals);
+                else
+                    hipLaunchKernelGGL(k_window_size_sort<512>, dim3((unsigned)nwin), dim3(kBlock), 0,
+                                       st, t->perm, t->sizes, n, (long long)rows, vals);
+                ok = hipGetLastError() == hipSuccess && count(vals, total);
+                if (ok && total.listed >= base && total.entries < best.entries) {
+                    best = total;
+                    t->sizeWindow = K;
+                    ok = hipMemcpyAsync(keep, vals, (size_t)rows * sizeof(int),
+                                        hipMemcpyDeviceToDevice, st) == hipSuccess;
+                }
+            }
+            if (ok && t->sizeWindow)
+                ok = hipMemcpyAsync(t->perm, keep, (size_t)rows * sizeof(int),
+                                    hipMemcpyDeviceToDevice, st) == hipSuccess;
+            if (ok) ok = count(t->perm, total);       // the counts of the kept order
+        }
     }
-    if (ok) t->listedSlices = listed;
     if (ok) {
-        t->sliceEntries = exclusive_scan(entries, t->sliceOff, S, st);
-        t->ctrlLen = exclusive_scan(listLen, t->ctrlOff, S, st);
-        ok = t->sliceEntries >= 0 && t->ctrlLen >= 0 &&
-             dalloc(&t->rec, (size_t)t->sliceEntries * rec_dwords(t->nw), t->bytes) &&
-             dalloc(&t->ctrl, (size_t)t->ctrlLen, t->bytes);
+        t->listedSlices = total.listed;
+        t->maxList = total.longest;
+        t->sliceEntries = total.entries;
+        t->ctrlLen = total.list;
+        ok = dalloc(&t->rec, (size_t)total.dwords, t->bytes) &&
+             dalloc(&t->ctrl, (size_t)total.list, t->bytes);
     }
     if (ok) {
-        if (t->nw == 1) OSDHIP_TILED(1, true, t->perm);
-        else if (t->nw == 3) OSDHIP_TILED(3, true, t->perm);
-        else OSDHIP_TILED(6, true, t->perm);
+        if (t->nw == 1) OSDHIP_COMPACT(1, true, t->perm);
+        else if (t->nw == 3) OSDHIP_COMPACT(3, true, t->perm);
+        else OSDHIP_COMPACT(6, true, t->perm);
         ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(st) == hipSuccess;
     }
-#undef OSDHIP_TILED
-    void *tmp[] = { keys, keysOut, vals, entries, listLen, sortTmp };
-    for (void *p : tmp)
-        if (p) (void)hipFree(p);
+#undef OSDHIP_COMPACT
+    (void)hipFree(scratch);
     return ok;
 }
 
@@ -519,8 +512,8 @@ osdhip_stencil_table *osdhip_stencil_table_create_ex(int numStencils, const int 
     void *scanTmp = nullptr;
     size_t scanBytes = 0;
     long long dummy = 0;
-    if (ok && S > 0 && t->layout == 2) {
-        ok = build_tiled(t, st);
+    if (ok && S > 0 && (t->layout == 0 || t->layout == 2)) {
+        ok = build_compact(t, st);
     } else if (ok && S > 0) {
         ok = dalloc(&t->sliceOff, (size_t)S, t->bytes) && dalloc(&t->sliceWidth, (size_t)S, t->bytes) &&
              dalloc(&t->rowSize, (size_t)rows, t->bytes) && dalloc(&entries, (size_t)S, dummy);
@@ -552,22 +545,6 @@ osdhip_stencil_table *osdhip_stencil_table_create_ex(int numStencils, const int 
                 hipLaunchKernelGGL(k_fill_records_paired, dim3(gr), dim3(kBlock), 0, st, t->sizes,
                                    t->offsets, t->indices, W[0], numStencils, rows, t->sliceOff,
                                    t->sliceWidth, t->rec);
-        } else if (ok && t->layout == 0) {
-            ok = dalloc(&t->rec, (size_t)t->sliceEntries * rec_dwords(numWeightArrays), t->bytes);
-            if (ok) {
-                if (numWeightArrays == 1)
-                    hipLaunchKernelGGL(k_fill_records<1>, dim3(gr), dim3(kBlock), 0, st, t->sizes,
-                                       t->offsets, t->indices, W[0], W[1], W[2], W[3], W[4], W[5],
-                                       numStencils, rows, t->sliceOff, t->sliceWidth, t->rec);
-                else if (numWeightArrays == 3)
-                    hipLaunchKernelGGL(k_fill_records<3>, dim3(gr), dim3(kBlock), 0, st, t->sizes,
-                                       t->offsets, t->indices, W[0], W[1], W[2], W[3], W[4], W[5],
-                                       numStencils, rows, t->sliceOff, t->sliceWidth, t->rec);
-                else
-                    hipLaunchKernelGGL(k_fill_records<6>, dim3(gr), dim3(kBlock), 0, st, t->sizes,
-                                       t->offsets, t->indices, W[0], W[1], W[2], W[3], W[4], W[5],
-                                       numStencils, rows, t->sliceOff, t->sliceWidth, t->rec);
-            }
         } else if (ok) {
             ok = dalloc(&t->sidx, (size_t)t->sliceEntries, t->bytes);
             for (int k = 0; ok && k < numWeightArrays; ++k)
@@ -695,53 +672,23 @@ int osdhip_stencil_table_eval(const osdhip_stencil_table *t, const float *src,
     const int nblocks = (nslices + kWavesPerBlock - 1) / kWavesPerBlock;
     const int grid = grid_for_blocks(nblocks);
     hipStream_t st = (hipStream_t)stream;
-    if (t->layout == 2) {
-        // a row range maps to slices anywhere in the locality order: every
-        // slice is visited and rows outside [start, end) are not written
-        TiledArgs a;
+    if (t->layout == 0 || t->layout == 2) {
+        CompactArgs a;
         std::memset(&a, 0, sizeof(a));
         a.srcStride = srcDesc.stride;
         a.perm = t->perm;
-        a.nuniq = t->nuniq;
-        a.ctrlOff = t->ctrlOff;
+        a.slices = t->slices;
         a.ctrl = t->ctrl;
-        a.sliceOff = t->sliceOff;
-        a.sliceWidth = t->sliceWidth;
         a.rec = t->rec;
+        a.slots = t->maxList + 1;
         a.rowBegin = start;
         a.rowEnd = end;
-        a.nslices = t->nslices;
-        a.nblocks = (t->nslices + kWavesPerBlock - 1) / kWavesPerBlock;
-        const int tgrid = grid_for_blocks(a.nblocks);
-        for (int e0 = 0; e0 < srcDesc.length; e0 += 8) {
-            const int lc = std::min(8, srcDesc.length - e0);
-            a.src = src + srcDesc.offset + e0;
-            for (int k = 0; k < numOutputs; ++k) {
-                a.dst[k] = outputs[k] ? outputs[k] + outputDescs[k].offset + e0 : nullptr;
-                a.dstStride[k] = outputs[k] ? outputDescs[k].stride : 0;
-            }
-            const int g = t->group == 4 ? 4 : 8;
-            if (t->nw == 1) launch_tiled<1>(lc, g, a, tgrid, st);
-            else if (t->nw == 3) launch_tiled<3>(lc, g, a, tgrid, st);
-            else launch_tiled<6>(lc, g, a, tgrid, st);
-            int rc = last_error();
-            if (rc != OSDHIP_OK) return rc;
-        }
-        return OSDHIP_OK;
-    }
-    if (t->layout == 0) {
-        RecArgs a;
-        std::memset(&a, 0, sizeof(a));
-        a.srcStride = srcDesc.stride;
-        a.rowSize = t->rowSize;
-        a.sliceOff = t->sliceOff;
-        a.sliceWidth = t->sliceWidth;
-        a.rec = t->rec;
-        a.rowBegin = start;
-        a.rowEnd = end;
-        a.sliceBegin = sliceBegin;
-        a.nslices = nslices;
-        a.nblocks = nblocks;
+        // in a locality order a row range maps to slices anywhere: every
+        // slice is visited and rows outside [start, end) are not written
+        a.sliceBegin = t->perm ? 0 : sliceBegin;
+        a.nslices = t->perm ? t->nslices : nslices;
+        a.nblocks = (a.nslices + kWavesPerBlock - 1) / kWavesPerBlock;
+        const int cgrid = grid_for_blocks(a.nblocks);
         for (int e0 = 0; e0 < srcDesc.length; e0 += 8) {
             const int lc = std::min(8, srcDesc.length - e0);
             a.src = src + srcDesc.offset + e0;
@@ -751,9 +698,9 @@ int osdhip_stencil_table_eval(const osdhip_stencil_table *t, const float *src,
             }
             // the kernel computes every weight array of the table; only the
             // requested outputs are written
-            if (t->nw == 1) launch_rec<1>(lc, t->group, a, grid, st);
-            else if (t->nw == 3) launch_rec<3>(lc, t->group, a, grid, st);
-            else launch_rec<6>(lc, t->group, a, grid, st);
+            if (t->nw == 1) launch_compact<1>(lc, a, cgrid, st);
+            else if (t->nw == 3) launch_compact<3>(lc, a, cgrid, st);
+            else launch_compact<6>(lc, a, cgrid, st);
             int rc = last_error();
             if (rc != OSDHIP_OK) return rc;
         }

@@ -4,6 +4,8 @@
 
 #include "../../include/osdhip.h"
 
+namespace osdhip { struct SliceDesc; }
+
 // Device copy of a (limit) stencil table: the Far CSR arrays (for the raw
 // getters) plus the 64-row slice layout the table kernels stream, built on
 // the device from the CSR arrays.
@@ -17,28 +19,24 @@ struct osdhip_stencil_table {
     long long nnz = 0, sliceEntries = 0, bytes = 0;
     int *sizes = nullptr, *offsets = nullptr, *indices = nullptr;
     float *w[6] = {};
+    // layouts 0 and 2: compact slices (stencil_compact.h)
+    osdhip::SliceDesc *slices = nullptr;
+    int *perm = nullptr;             // slice row -> Far row (>= n: padding); NULL: Far's order
+    int *ctrl = nullptr;             // control lists
+    long long ctrlLen = 0;
+    int maxList = 0;                 // longest control list
+    unsigned *rec = nullptr;         // stored entries; layout 3: paired records
+    // layouts 1 and 3
     long long *sliceOff = nullptr;
     int *sliceWidth = nullptr;
     int *rowSize = nullptr;          // sizes padded to nslices * 64 rows
-    unsigned *rec = nullptr;         // layouts 0, 2: records of rec_dwords(nw)
     int *sidx = nullptr;             // layout 1: split streams
     float *sw[6] = {};
-    // layout 2 (locality-ordered slices): slice row i holds Far row perm[i]
-    // (>= n: padding); a slice with nuniq[s] >= 0 lists its distinct control
-    // vertices at ctrl[ctrlOff[s] ...] and its records hold positions in
-    // that list; nuniq[s] < 0: records hold control indices
-    int *perm = nullptr;
-    int *nuniq = nullptr;
-    long long *ctrlOff = nullptr;
-    int *ctrl = nullptr;
-    long long ctrlLen = 0;
     int listedSlices = 0;
     int sizeWindow = 0;              // layout 2, order 0: rows sorted by size per window (0: none)
 };
 
 namespace osdhip {
-
-inline int rec_dwords(int nw) { return nw == 1 ? 2 : nw == 3 ? 4 : 8; }
 
 inline int last_error()
 {

@@ -2,8 +2,8 @@
 // uploaded CSR arrays (used by osdhip_stencil_table_create only).
 #pragma once
 #include "common.h"
+#include "stencil_compact.h"
 #include "stencil_sliced.h"
-#include "stencil_tiled.h"
 
 namespace osdhip {
 
@@ -29,36 +29,6 @@ __global__ __launch_bounds__(kBlock) void k_pad_sizes(const int *sizes, int n, i
     const int r = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (r >= rows) return;
     padded[r] = r < n ? sizes[r] : 0;
-}
-
-// One lane per slice row: writes the row's W records (padding included).
-template <int NWT>
-__global__ __launch_bounds__(kBlock) void k_fill_records(
-    const int *sizes, const int *offsets, const int *indices, const float *w0, const float *w1,
-    const float *w2, const float *w3, const float *w4, const float *w5, int n, int rows,
-    const long long *sliceOff, const int *sliceWidth, unsigned *rec)
-{
-    constexpr int R = RecShape<NWT>::R;
-    const int r = (int)(blockIdx.x * kBlock + threadIdx.x);
-    if (r >= rows) return;
-    const int s = r / kWave, lane = r % kWave;
-    const int W = sliceWidth[s];
-    const int sz = r < n ? sizes[r] : 0;
-    const long long off = r < n ? (long long)offsets[r] : 0;
-    const float *ws[6] = { w0, w1, w2, w3, w4, w5 };
-    for (int j = 0; j < W; ++j) {
-        unsigned q[R];
-#pragma unroll
-        for (int k = 0; k < R; ++k) q[k] = 0u;
-        if (j < sz) {
-            q[0] = (unsigned)indices[off + j];
-#pragma unroll
-            for (int k = 0; k < NWT; ++k) q[1 + k] = __float_as_uint(ws[k][off + j]);
-        }
-        unsigned *d = rec + (size_t)(sliceOff[s] + (long long)j * kWave + lane) * R;
-#pragma unroll
-        for (int k = 0; k < R; ++k) d[k] = q[k];
-    }
 }
 
 // Paired records (one weight array): entries 2p and 2p + 1 of a row sit
@@ -88,8 +58,8 @@ __global__ __launch_bounds__(kBlock) void k_fill_records_paired(
     }
 }
 
-// Split-stream layout (index and each weight array in its own column-major
-// slice stream), kept as an alternative for the autotuner.
+// Split-stream layout (layout 1: index and each weight array in its own
+// column-major slice stream).
 __global__ __launch_bounds__(kBlock) void k_fill_split(
     const int *sizes, const int *offsets, const int *indices, const float *w0, const float *w1,
     const float *w2, const float *w3, const float *w4, const float *w5, int nw, int n, int rows,
@@ -112,33 +82,27 @@ __global__ __launch_bounds__(kBlock) void k_fill_split(
 }
 
 // ---------------------------------------------------------------------------
-// Locality-ordered slices (layout 2).
+// Compact slices (layouts 0 and 2; stencil_compact.h).
 //
-// Rows are ordered by their dominant control vertex (the entry of largest
-// |weight|, the first one on ties; a stable sort keeps Far order among
-// equal keys), so the 64 rows of a slice surround a few control vertices and
-// share most of their support: 26-38 distinct control vertices per slice on
-// creased cube-spheres at levels 2-4, against 30 (level 4) to 100 (level 2)
-// on average in Far order -- which keeps a slice's 64 outputs consecutive
-// (order option 1).  Per slice
-// the distinct control vertices are listed in ascending order; when there
-// are at most kTileZero of them the slice's records hold list positions
-// (LDS slots), otherwise control indices.
+// Layout 0 keeps Far's row order.  Layout 2's locality order sorts rows by
+// their dominant control vertex (the entry of largest |weight|, the first
+// one on ties; a stable sort keeps Far order among equal keys), so the 64
+// rows of a slice surround a few control vertices and share most of their
+// support: 26-38 distinct control vertices per slice on creased
+// cube-spheres at levels 2-4, against 30 (level 4) to 100 (level 2) on
+// average in Far order -- which keeps a slice's 64 outputs consecutive.
 
-// Sort key per slice row: the dominant control vertex (empty rows:
-// 0xffffffff), or with farOrder the row itself (Far's order kept); rows
-// past n: 0xffffffff, after every real key; value: the row.
+// Sort key per slice row: the dominant control vertex (empty rows and rows
+// past n: 0xffffffff; the sort is stable, so padding stays last); value:
+// the row.
 __global__ __launch_bounds__(kBlock) void k_row_dominant(const int *sizes, const int *offsets,
                                                          const int *indices, const float *w0, int n,
-                                                         int rows, int farOrder, unsigned *keys,
-                                                         int *vals)
+                                                         int rows, unsigned *keys, int *vals)
 {
     const int r = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (r >= rows) return;
     unsigned key = 0xffffffffu;
-    if (farOrder) {
-        if (r < n) key = (unsigned)r;
-    } else if (r < n && sizes[r] > 0) {
+    if (r < n && sizes[r] > 0) {
         const long long off = offsets[r];
         key = (unsigned)indices[off];
         float best = fabsf(w0[off]);
@@ -193,88 +157,155 @@ __global__ __launch_bounds__(kBlock) void k_window_size_sort(const int *in, cons
     }
 }
 
-// One wave per slice of the ordered rows perm[].  Count pass (FILL false):
-// slice width, record entries (64 * width), distinct control vertices
-// (nuniq = -1 when more than kTileZero) and list length.  Fill pass: the
-// ascending control list and the records -- {list position, weights} for a
-// listed slice (padding: {kTileZero, 0}), {control index, weights} otherwise
-// (padding: {kTilePad, 0}).  Distinct vertices are extracted in ascending
-// order by repeated wave minima over the slice's entries.
+// Open-addressed set of a slice's control indices in LDS.  A slice stops
+// inserting once more than `cap` <= kSliceList are distinct, so at most
+// kSliceList + 64 of the kSetSize places are ever taken and every probe
+// ends at a free place or its own key.
+constexpr int kSetSize = 512;
+static_assert(kSliceList + kWave < kSetSize, "probes end");
+__device__ __forceinline__ int set_home(unsigned x) { return (int)((x * 2654435761u) >> 23); }
+
+// True when x was not in the set yet.
+__device__ __forceinline__ bool set_insert(unsigned *h, unsigned x)
+{
+    for (int p = set_home(x);; p = (p + 1) & (kSetSize - 1)) {
+        const unsigned old = atomicCAS(h + p, kSliceNoIndex, x);
+        if (old == kSliceNoIndex) return true;
+        if (old == x) return false;
+    }
+}
+
+__device__ __forceinline__ int set_find(const unsigned *h, unsigned x)
+{
+    int p = set_home(x);
+    while (h[p] != x) p = (p + 1) & (kSetSize - 1);
+    return p;
+}
+
+// What the slices before one hold (an exclusive scan) and what one holds.
+struct SliceCount {
+    long long entries;      // 64 * width
+    long long dwords;       // stored entries
+    long long list;         // listed control vertices
+    int listed;             // 1: the slice lists its control vertices
+    int longest;            // longest list (a maximum, not a sum)
+};
+struct SliceCountAdd {
+    __host__ __device__ SliceCount operator()(const SliceCount &a, const SliceCount &b) const
+    {
+        return { a.entries + b.entries, a.dwords + b.dwords, a.list + b.list, a.listed + b.listed,
+                 a.longest > b.longest ? a.longest : b.longest };
+    }
+};
+
+// One wave per slice of the ordered rows perm[] (NULL: Far's order).  Count
+// pass (FILL false): slice width, distinct control vertices (nuniq = -1 when
+// more than `cap`) and what it holds.  Fill pass: the descriptor, the ascending control
+// list, the slot bytes (or control indices) and the weights, as
+// stencil_compact.h lays them out.
 template <int NWT, bool FILL>
-__global__ __launch_bounds__(kBlock) void k_tiled_slices(
+__global__ __launch_bounds__(kBlock) void k_compact_slices(
     const int *perm, const int *sizes, const int *offsets, const int *indices, const float *w0,
     const float *w1, const float *w2, const float *w3, const float *w4, const float *w5, int n, int S,
-    int *width, long long *entries, int *nuniq, long long *listLen, const long long *sliceOff,
-    const long long *ctrlOff, int *ctrl, unsigned *rec)
+    int cap, int *width, int *nuniq, SliceCount *counts, const SliceCount *before,
+    SliceDesc *slices, int *ctrl, unsigned *rec)
 {
-    constexpr int R = RecShape<NWT>::R;
+    __shared__ unsigned set[kWavesPerBlock][kSetSize];
+    __shared__ unsigned char rank[FILL ? kWavesPerBlock : 1][kSetSize];
+    __shared__ unsigned vals[FILL ? kWavesPerBlock : 1][kSliceList];
+    __shared__ unsigned short place[FILL ? kWavesPerBlock : 1][kSliceList];
     const int lane = (int)threadIdx.x & (kWave - 1);
-    const int s = (int)blockIdx.x * kWavesPerBlock + wave_in_block();
+    const int wv = wave_in_block();
+    const int s = (int)blockIdx.x * kWavesPerBlock + wv;
     if (s >= S) return;                                // whole wave
-    const int r = perm[(long long)s * kWave + lane];
+    unsigned *h = set[wv];
+    const long long i = (long long)s * kWave + lane;
+    const int r = perm ? perm[i] : (int)min(i, (long long)n);
     const bool valid = r >= 0 && r < n;
     const int sz = valid ? sizes[r] : 0;
     const long long off = valid ? (long long)offsets[r] : 0;
-    const float *ws[6] = { w0, w1, w2, w3, w4, w5 };
     const int W = FILL ? width[s] : wave_max_i(sz);
-    const bool listed = FILL ? nuniq[s] >= 0 : true;
-    unsigned *rp = FILL ? rec + (size_t)(sliceOff[s] + lane) * R : nullptr;
-    int U = 0;
-    bool over = false;
-    if (listed) {
-        long long last = -1;
-        for (;;) {
-            unsigned m = 0xffffffffu;
-            for (int j = 0; j < sz; ++j) {
+    int U = FILL ? nuniq[s] : 0;
+    if (!FILL || U >= 0) {
+        for (int k = lane; k < kSetSize; k += kWave) h[k] = kSliceNoIndex;
+        wave_lds_sync();
+        int found = 0;
+        bool over = false;
+        for (int j = 0; j < W && !over; ++j) {         // wave-uniform
+            bool fresh = false, bad = false;
+            if (j < sz) {
                 const unsigned x = (unsigned)indices[off + j];
-                if ((long long)x > last) m = min(m, x);
+                bad = x == kSliceNoIndex;              // the free mark: such a slice is not listed
+                if (!bad) fresh = set_insert(h, x);
             }
-            m = wave_min_u(m);
-            if (m == 0xffffffffu) break;
-            if (U == kTileZero) {
-                over = true;
-                break;
-            }
-            if (FILL) {
-                if (lane == 0) ctrl[ctrlOff[s] + U] = (int)m;
-                for (int j = 0; j < sz; ++j) {
-                    if ((unsigned)indices[off + j] != m) continue;
-                    unsigned *d = rp + (size_t)j * (kWave * R);
-                    d[0] = (unsigned)U;
-#pragma unroll
-                    for (int k = 0; k < NWT; ++k) d[1 + k] = __float_as_uint(ws[k][off + j]);
-#pragma unroll
-                    for (int k = 1 + NWT; k < R; ++k) d[k] = 0u;
-                }
-            }
-            last = m;
-            ++U;
+            found += __popcll(__ballot(fresh));
+            over = found > cap || __ballot(bad) != 0;
         }
+        if (!FILL) U = over ? -1 : found;
     }
     if (!FILL) {
         if (lane == 0) {
             width[s] = W;
-            entries[s] = (long long)W * kWave;
-            nuniq[s] = over ? -1 : U;
-            listLen[s] = over ? 0 : U;
+            nuniq[s] = U;
+            counts[s] = { (long long)W * kWave,
+                          (long long)slice_index_dwords(W, U) + (long long)W * NWT * kWave,
+                          max(U, 0), U >= 0, max(U, 0) };
         }
         return;
     }
-    for (int j = 0; j < W; ++j) {
-        unsigned *d = rp + (size_t)j * (kWave * R);
-        if (listed && j < sz) continue;                // written above
-        unsigned q[R];
-#pragma unroll
-        for (int k = 0; k < R; ++k) q[k] = 0u;
-        if (j < sz) {
-            q[0] = (unsigned)indices[off + j];
-#pragma unroll
-            for (int k = 0; k < NWT; ++k) q[1 + k] = __float_as_uint(ws[k][off + j]);
-        } else {
-            q[0] = listed ? (unsigned)kTileZero : kTilePad;
+    const long long recOff = before[s].dwords, ctrlOff = before[s].list;
+    if (lane == 0) {
+        SliceDesc d;
+        d.off = recOff;
+        d.ctrlOff = ctrlOff;
+        d.width = W;
+        d.nuniq = U;
+        d.pad[0] = d.pad[1] = 0;
+        slices[s] = d;
+    }
+    if (U >= 0) {
+        // the set's members side by side, then each one's rank among them
+        wave_lds_sync();
+        int count = 0;
+        for (int k = 0; k < kSetSize; k += kWave) {
+            const unsigned x = h[k + lane];
+            const unsigned long long m = __ballot(x != kSliceNoIndex);
+            if (x != kSliceNoIndex) {
+                const int at = count + __popcll(m & ((1ull << lane) - 1));
+                vals[wv][at] = x;
+                place[wv][at] = (unsigned short)(k + lane);
+            }
+            count += __popcll(m);
         }
+        wave_lds_sync();
+        for (int k = lane; k < U; k += kWave) {
+            const unsigned x = vals[wv][k];
+            int below = 0;
+            for (int q = 0; q < U; ++q) below += vals[wv][q] < x;
+            rank[wv][place[wv][k]] = (unsigned char)below;
+            ctrl[ctrlOff + below] = (int)x;
+        }
+        wave_lds_sync();
+    }
+    unsigned *rp = rec + recOff;
+    float *wp = (float *)(rp + slice_index_dwords(W, U));
+    const float *ws[6] = { w0, w1, w2, w3, w4, w5 };
+    for (int g = 0; 4 * g < W; ++g) {
+        unsigned bytes = 0u;
+        const int left = min(4, W - 4 * g);            // wave-uniform
+        for (int u = 0; u < 4; ++u) {
+            const int j = 4 * g + u;
+            const bool in = j < sz;
+            const unsigned x = in ? (unsigned)indices[off + j] : kSliceNoIndex;
+            if (U >= 0) bytes |= (in ? (unsigned)rank[wv][set_find(h, x)] : (unsigned)U) << (8 * u);
+            if (u >= left) continue;
+            if (U < 0) rp[(size_t)j * kWave + lane] = x;
+            float *d = NWT == 1 ? wp + (size_t)g * (4 * kWave) + left * lane + u
+                                : wp + (size_t)j * (NWT * kWave) + NWT * lane;
 #pragma unroll
-        for (int k = 0; k < R; ++k) d[k] = q[k];
+            for (int k = 0; k < NWT; ++k) d[k] = in ? ws[k][off + j] : 0.0f;
+        }
+        if (U >= 0) rp[(size_t)g * kWave + lane] = bytes;
     }
 }
 

@@ -119,13 +119,14 @@ class HipStencilTable:
     a dict with keys sizes/offsets/indices/weights[/du/dv/duu/duv/dvv].
 
     Device options (osdhip_table_options, fixed per table): ``layout`` 0
-    (record slices), 1 (split streams) or 2 (locality-ordered slices staged
-    in LDS); ``keep_csr`` keeps the Far CSR arrays on the device; ``group``
+    (compact slices in Far's row order), 1 (split streams), 2 (compact slices
+    in a locality order) or 3 (paired records, one weight array); ``keep_csr`` keeps the Far CSR arrays on the device; ``group``
     (4, 8, 16) and ``kernel`` (0 slices, 1 CSR) select the evaluation
     kernel and can be changed later with ``set``; ``order`` (layout 2) 0
     groups rows by dominant control vertex and then by size within row
     windows when that streams fewer padded entries, 2 by dominant control
-    vertex only, 1 keeps Far's row order."""
+    vertex only (Far's order for large tables whose slices list few control
+    vertices in it), 1 keeps Far's row order."""
 
     _KEYS = ["weights", "du", "dv", "duu", "duv", "dvv"]
     _GETTERS = ["GetWeights", "GetDuWeights", "GetDvWeights", "GetDuuWeights",

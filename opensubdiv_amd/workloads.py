@@ -208,11 +208,12 @@ class DeviceMesh:
         self.out = None
         if own_outputs:
             self.bind_outputs(torch.empty(self.output_floats(), dtype=torch.float32, device=dev))
-        # stencil tables in slice layout `layout` (0 record slices, 2
-        # locality-ordered, rows by dominant vertex (order 2: a slice's
-        # control vertices are staged once per frame chunk, so fewer of them
-        # beats the fewer padded entries of order 0's size windows), or in
-        # Far's order (order 1)); the batch kernels need no CSR arrays
+        # stencil tables in slice layout `layout` (0 Far's row order, 2
+        # locality-ordered: order 2, rows by dominant vertex, or Far's order
+        # where its slices list few control vertices (a slice's control
+        # vertices are staged once per frame chunk, so fewer of them beats
+        # the fewer padded entries of order 0's size windows); or order 1,
+        # Far's order); the batch kernels need no CSR arrays
         self.refine_table = HipStencilTable(h.refine, stream, layout=layout, keep_csr=keep_csr,
                                             order=order)
         self.point_table = HipStencilTable(h.points, stream, layout=layout, keep_csr=keep_csr,
