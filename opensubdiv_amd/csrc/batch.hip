@@ -9,6 +9,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <climits>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -46,7 +47,7 @@ struct osdhip_batch {
     std::vector<int> beginA, countA;       // phase-A item ranges per stage
     // phase-B item ranges per (launch kind, stage): each launch visits only
     // the items with waves of its kind
-    std::vector<int> beginB[5], countB[5];
+    std::vector<int> beginB[5], countB[5], framesB[5];   // and an item's frames
     std::vector<std::vector<int>> hNuniq, hNgen;   // per patch segment, while building
     unsigned *counters = nullptr;          // kCounters per (stage, phase)
     int numCUs = 256;
@@ -117,13 +118,12 @@ template <int LC, int FC>
 void launchB(const PhaseB &L, bool staged, hipStream_t st)
 {
     if (staged) {
-        launchKind(L, kB_S128, k_batch_patches_regular<LC, FC, kStagedOnly, 128>, st);
-        // 256 slots one frame per chunk (LDS: 4 waves x FC x LC x 256 floats,
-        // 28 KB at LC 7, so LDS allows as many blocks per CU as registers do)
-        launchKind(L, kB_S256, k_batch_patches_regular<LC, 1, kStagedOnly, 256>, st);
-        launchKind(L, kB_Unl, k_batch_patches_regular<LC, FC, kGatherUnlisted>, st);
+        launchKind(L, kB_S128, k_batch_patches_staged<LC, FC, 128>, st);
+        // 256 slots one frame per chunk (LDS)
+        launchKind(L, kB_S256, k_batch_patches_staged<LC, 1, 256>, st);
+        launchKind(L, kB_Unl, k_batch_patches_gather<LC, FC, false>, st);
     } else {
-        launchKind(L, kB_All, k_batch_patches_regular<LC, FC, kGatherAll>, st);
+        launchKind(L, kB_All, k_batch_patches_gather<LC, FC, true>, st);
     }
     // the few other coords (Gregory, boundary, bilinear): one frame per chunk
     // keeps the general kernel's register budget lower
@@ -214,6 +214,23 @@ bool preparePatchStaging(osdhip_batch *b, BatchPatchSeg &g)
     return true;
 }
 
+// Frames per phase-B item: all of a coord's, unless the launch then has too
+// few blocks for the chip; fewer (16, 8, ... down to `least`, the frames a
+// kernel takes per chunk) until it has eight blocks per CU.  12 meshes of 679 K
+// coords, 1 to 16 frames: the general kernel 70 us with every frame in one
+// item, 14 us split; coords gathered from memory 205 and 160 us.
+int itemFrames(const osdhip_batch *b, const std::vector<BatchItem> &base, int least)
+{
+    int step = INT_MAX;
+    for (int g = 16; g >= least; g /= 2) {
+        long long blocks = 0;
+        for (const BatchItem &it : base) blocks += ((long long)b->hP[it.seg].frames + step - 1) / step;
+        if (blocks >= 8LL * b->numCUs) break;
+        step = g;
+    }
+    return step;
+}
+
 // (Re)builds the phase-A item list for cfg.aItemSlices.
 int buildItemsA(osdhip_batch *b)
 {
@@ -290,6 +307,7 @@ int enqueuePhaseB(osdhip_batch *b, int stage, hipStream_t st)
         a.pseg = b->dP;
         a.items = b->itemsB + b->beginB[k][stage];
         a.nitems = b->countB[k][stage];
+        a.itemFrames = b->framesB[k][stage];
         a.persistent = b->cfg.bPersistent;
         a.counter = b->counters + kCounters * (2 * stage + 1);
         L.grid[k] = gridFor(b, a.nitems, a.persistent != 0);
@@ -471,8 +489,9 @@ static osdhip_batch *batch_create(int length, int numStencilSegments,
     for (int k = 0; k < kBKinds; ++k) {
         b->beginB[k].assign(b->nStages, 0);
         b->countB[k].assign(b->nStages, 0);
+        b->framesB[k].assign(b->nStages, INT_MAX);
         for (int st = 0; st < b->nStages; ++st) {
-            b->beginB[k][st] = (int)itemsB.size();
+            std::vector<BatchItem> base;               // every frame in one item
             for (int seg = 0; seg < b->nP; ++seg) {
                 if (b->pStage[seg] != st) continue;
                 const int nc = b->hP[seg].ncoords;
@@ -484,9 +503,15 @@ static osdhip_batch *batch_create(int length, int numStencilSegments,
                              : k == kB_S256 ? nu[w] > 128
                              : k == kB_Unl ? nu[w] < 0
                              : ng[w] > 0;
-                    if (take) itemsB.push_back({ seg, c, std::min(kBlock, nc - c), 0 });
+                    if (take) base.push_back({ seg, c, std::min(kBlock, nc - c), 0 });
                 }
             }
+            const int step = itemFrames(b, base, k == kB_Gen ? 1 : 4);
+            b->framesB[k][st] = step;
+            b->beginB[k][st] = (int)itemsB.size();
+            for (const BatchItem &it : base)
+                for (long long f = 0; f < b->hP[it.seg].frames; f += step)
+                    itemsB.push_back({ it.seg, it.first, it.count, (int)f });
             b->countB[k][st] = (int)itemsB.size() - b->beginB[k][st];
         }
     }
@@ -955,6 +980,7 @@ int osdhip_batch_epoch(int length, int numStencilSegments, const osdhip_batch_st
             L.a[k].pseg = (const BatchPatchSeg *)(d + p.segB);
             L.a[k].items = (const BatchItem *)(d + p.itemsB);
             L.a[k].nitems = nb;
+            L.a[k].itemFrames = INT_MAX;
             L.grid[k] = grid_for_blocks(nb);
         }
         if (!launchB_variant(length, 1, false, L, st))

@@ -175,7 +175,8 @@ __device__ __forceinline__ osdhip_patch_param ld(const G_ osdhip_patch_param *p)
 }
 
 struct BatchItem {
-    int seg, first, count, pad;   // phase A: slices [first, first+count); B: coords
+    int seg, first, count;        // phase A: slices [first, first+count); B: coords
+    int f0;                       // phase B: first frame
 };
 
 __device__ __forceinline__ BatchItem ld(const C_ BatchItem *p)
@@ -184,7 +185,7 @@ __device__ __forceinline__ BatchItem ld(const C_ BatchItem *p)
     it.seg = p->seg;
     it.first = p->first;
     it.count = p->count;
-    it.pad = 0;
+    it.f0 = p->f0;
     return it;
 }
 
@@ -194,6 +195,7 @@ struct BatchArgs {
     const BatchItem *items;
     int nitems;
     int persistent;
+    int itemFrames;               // phase B: an item's frames are [f0, f0 + itemFrames)
     unsigned *counter;            // persistent: one claim counter per XCD queue
 };
 
@@ -623,13 +625,12 @@ __device__ __forceinline__ void batch_patch_point(const G_ float *p, long long f
     }
 }
 
-// Phase B in two kernels over the same items, each with its own register
-// budget:
-//   k_batch_patches_regular  regular B-spline patches without boundary (nearly
+// Phase B in kernels of their own register budgets:
+//   k_batch_patches_staged,
+//   k_batch_patches_gather   regular B-spline patches without boundary (nearly
 //                            all coords): the 16 weights are formed in-line
 //                            from the separable curves -- the same single
-//                            products basis_bspline stores -- one row of 4
-//                            points at a time, so few gathers are live;
+//                            products basis_bspline stores;
 //   k_batch_patches          every other coord (Gregory, boundary, bilinear),
 //                            skipping the regular-interior ones.
 __device__ __forceinline__ float pick4(const float (&v)[4], int r)
@@ -685,22 +686,76 @@ __device__ __forceinline__ void store_patch_chunk(const GPatchSeg &sg, int i, in
     }
 }
 
-// Waves of 64 coords in three modes, each launch with its own register
-// budget: kGatherAll gathers every regular coord's points from memory;
-// kStagedOnly takes the waves whose coords reference at most kPatchSlots
-// distinct points (listed by k_patch_slots): the wave copies those points'
-// frames into LDS -- element (q, k) of slot u at lds[q * LC + k][u], one or
-// two slots per lane -- and reads each coord's 16 points from LDS through
-// its slot bytes; kGatherUnlisted gathers for the other waves.  Same
-// products and order in every mode.
-enum { kGatherAll = 0, kStagedOnly = 1, kGatherUnlisted = 2 };
-
-template <int LC, int FC, int MODE, int SLOTS = 128>
-__global__ __launch_bounds__(kBlock) void k_batch_patches_regular(BatchArgs a)
+// Regular coords of waves that are not staged (k_batch_patches_gather: every
+// wave with ALL, else those whose list is longer than kPatchSlots) gather
+// their points from memory; k_batch_patches_staged takes the waves whose
+// coords reference at most SLOTS distinct points (listed by k_patch_slots).
+// Same products and order in both.  An item takes itemFrames frames of its
+// coords: small batches split a coord's frames over several items, because
+// one wave's frames follow one another at a load latency each.
+template <int LC, int FC, bool ALL>
+__global__ __launch_bounds__(kBlock) void k_batch_patches_gather(BatchArgs a)
 {
-    constexpr bool STAGED = MODE == kStagedOnly;
-    __shared__ float lds[STAGED ? kWavesPerBlock : 1][STAGED ? FC * LC : 1][STAGED ? SLOTS : 1];
-    const int lane = (int)threadIdx.x & (kWave - 1);
+    const int wv = wave_in_block();
+    for (int iter = 0;; ++iter) {
+        const int itx = batch_next_item(a, iter);
+        if (itx < 0) break;
+        const BatchItem item = ld(cptr(a.items) + itx);
+        const GPatchSeg sg = gseg(cptr(a.pseg)[item.seg]);
+        const int i = item.first + (int)threadIdx.x;
+        if (i >= item.first + item.count) continue;
+        // the wave's entry in the staging lists (items start at multiples of
+        // kBlock coords; a wave past the segment's end has none)
+        if (!ALL && sg.nuniq && sg.nuniq[(item.first >> 6) + wv] >= 0) continue;
+        const RegularCoord rc = regular_coord(sg, i);
+        if (!rc.ok) continue;
+        Curve cs, ct;
+        bspline_curve(rc.s, cs);
+        bspline_curve(rc.t, ct);
+        const int fEnd = item.f0 + min(a.itemFrames, sg.frames - item.f0);
+        for (int f0 = item.f0; f0 < fEnd; f0 += FC) {
+            const int nq = min(FC, fEnd - f0);
+            float acc[3][FC][LC];
+#pragma unroll
+            for (int o = 0; o < 3; ++o)
+#pragma unroll
+                for (int q = 0; q < FC; ++q)
+#pragma unroll
+                    for (int k = 0; k < LC; ++k) acc[o][q][k] = 0.0f;
+            const G_ float *base = sg.src + (size_t)f0 * sg.srcF;
+#pragma unroll 1
+            for (int r = 0; r < 4; ++r) {                 // point j = 4 r + q
+                const float tb = pick4(ct.b, r), td = pick4(ct.d, r);
+                int idx[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) idx[q] = rc.cvs[4 * r + q];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    batch_patch_point<LC, FC>(base + (size_t)(unsigned)idx[q] * sg.srcV, sg.srcF,
+                                              nq, cs.b[q] * tb, cs.d[q] * tb, cs.b[q] * td, acc);
+            }
+            store_patch_chunk<LC, FC>(sg, i, f0, nq, rc.k1, acc);
+        }
+    }
+}
+
+// Staged waves: the wave copies its listed points' FC frames into LDS, each
+// lane one 16-byte quad of one (point, frame) as k_batch_stencils does, and
+// every lane reads its coord's 16 points through its slot bytes with 16-byte
+// reads (slot-major, as BatchChunk pads them).  12 meshes of 679 K coords, 1
+// to 16 frames of 7 floats, with the frames of a coord split over items:
+// lists up to 128 172 -> 146 us, longer lists 119 -> 70 us against one point
+// per lane and value-major 4-byte reads (2.0 TB/s of output).
+template <int LC, int FC, int SLOTS>
+__global__ __launch_bounds__(kBlock) void k_batch_patches_staged(BatchArgs a)
+{
+    using A = BatchChunk<LC, FC>;
+    constexpr int STR = A::STR;
+    constexpr int H = (LC + 3) / 4;                       // quads per (point, frame)
+    constexpr int N = LC < 4 ? LC : 4;                    // floats per copied quad
+    constexpr int QP = FC * H;                            // quads per point: 1, 2, 4 or 8
+    constexpr int PI = kWave / QP;                        // points per copy instruction
+    __shared__ __attribute__((aligned(16))) float lds[kWavesPerBlock][SLOTS * STR];
     const int wv = wave_in_block();
     for (int iter = 0;; ++iter) {
         const int itx = batch_next_item(a, iter);
@@ -711,49 +766,14 @@ __global__ __launch_bounds__(kBlock) void k_batch_patches_regular(BatchArgs a)
         const bool inRange = i < item.first + item.count;
         // the wave's entry in the staging lists (items start at multiples of
         // kBlock coords); a wave past the segment's end has none
-        const bool waveHasCoords = wv * kWave < item.count;
-        const int U = (MODE != kGatherAll && sg.nuniq && waveHasCoords)
-                          ? sg.nuniq[(item.first >> 6) + wv] : -1;
-        // staged variants: 128 slots take U <= 128, 256 slots 128 < U <= 256
-        if (MODE == kStagedOnly && (U < 0 || U > SLOTS || (SLOTS > 128 && U <= 128))) continue;
-        if (MODE == kGatherUnlisted && U >= 0) continue;
+        const int U = wv * kWave < item.count ? sg.nuniq[(item.first >> 6) + wv] : -1;
+        // 128 slots take U <= 128, 256 slots 128 < U <= 256
+        if (U < 0 || U > SLOTS || (SLOTS > 128 && U <= 128)) continue;
 
-        if (!STAGED) {                                    // gathers from memory
-            if (!inRange) continue;
-            const RegularCoord rc = regular_coord(sg, i);
-            if (!rc.ok) continue;
-            Curve cs, ct;
-            bspline_curve(rc.s, cs);
-            bspline_curve(rc.t, ct);
-            for (int f0 = 0; f0 < sg.frames; f0 += FC) {
-                const int nq = min(FC, sg.frames - f0);
-                float acc[3][FC][LC];
-#pragma unroll
-                for (int o = 0; o < 3; ++o)
-#pragma unroll
-                    for (int q = 0; q < FC; ++q)
-#pragma unroll
-                        for (int k = 0; k < LC; ++k) acc[o][q][k] = 0.0f;
-                const G_ float *base = sg.src + (size_t)f0 * sg.srcF;
-#pragma unroll 1
-                for (int r = 0; r < 4; ++r) {             // point j = 4 r + q
-                    const float tb = pick4(ct.b, r), td = pick4(ct.d, r);
-                    int idx[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) idx[q] = rc.cvs[4 * r + q];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        batch_patch_point<LC, FC>(base + (size_t)(unsigned)idx[q] * sg.srcV,
-                                                  sg.srcF, nq, cs.b[q] * tb, cs.d[q] * tb,
-                                                  cs.b[q] * td, acc);
-                }
-                store_patch_chunk<LC, FC>(sg, i, f0, nq, rc.k1, acc);
-            }
-            continue;
-        }
-
-        // staged wave: every lane takes part in the copies
-        float(*Ls)[STAGED ? SLOTS : 1] = lds[STAGED ? wv : 0];
+        // every lane takes part in the copies
+        float *area = lds[wv];
+        const int lane = lane_here();
+        const G_ int *lst = sg.pts + sg.ptsOff[(item.first >> 6) + wv];
         RegularCoord rc;
         rc.ok = false;
         if (inRange) rc = regular_coord(sg, i);
@@ -765,26 +785,30 @@ __global__ __launch_bounds__(kBlock) void k_batch_patches_regular(BatchArgs a)
         Curve cs, ct;
         bspline_curve(rc.ok ? rc.s : 0.0f, cs);
         bspline_curve(rc.ok ? rc.t : 0.0f, ct);
-        const G_ int *lst = sg.pts + sg.ptsOff[(item.first >> 6) + wv];
-        constexpr int PER = STAGED ? SLOTS / kWave : 1;   // slots per lane
-        int vv[PER];
-#pragma unroll
-        for (int h = 0; h < PER; ++h) vv[h] = lane + h * kWave < U ? lst[lane + h * kWave] : 0;
-        for (int f0 = 0; f0 < sg.frames; f0 += FC) {
-            const int nq = min(FC, sg.frames - f0);
+        // this lane's quad of its points: frame c of the chunk, floats
+        // [k0, k0 + N) (the last quad of 5 to 7 floats overlaps the one before)
+        const int q = lane % QP, c = q / H, k0 = min(4 * (q % H), LC - N);
+        const int fEnd = item.f0 + min(a.itemFrames, sg.frames - item.f0);
+        for (int f0 = item.f0; f0 < fEnd; f0 += FC) {
+            const int nq = min(FC, fEnd - f0);
             wave_lds_sync();                              // previous chunk's reads are done
+            const G_ float *p = sg.src + (size_t)(f0 + min(c, nq - 1)) * sg.srcF + k0;
+            for (int u0 = 0; u0 < U; u0 += 4 * PI) {      // four copies in flight
+                float x[4][N];
+                int pt[4];
 #pragma unroll
-            for (int h = 0; h < PER; ++h) {
-                const int u = lane + h * kWave;
-                if (u < U) {
-                    const G_ float *p = sg.src + (size_t)(unsigned)vv[h] * sg.srcV +
-                                        (size_t)f0 * sg.srcF;
+                for (int r = 0; r < 4; ++r) pt[r] = lst[min(u0 + r * PI + lane / QP, U - 1)];
 #pragma unroll
-                    for (int q = 0; q < FC; ++q) {
-                        if (q < nq) {                     // wave-uniform
+                for (int r = 0; r < 4; ++r)
 #pragma unroll
-                            for (int k = 0; k < LC; ++k) Ls[q * LC + k][u] = p[q * sg.srcF + k];
-                        }
+                    for (int k = 0; k < N; ++k) x[r][k] = p[(size_t)(unsigned)pt[r] * sg.srcV + k];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int u = u0 + r * PI + lane / QP;
+                    if (u < U) {
+                        float *d = area + u * STR + c * LC + k0;
+#pragma unroll
+                        for (int k = 0; k < N; ++k) d[k] = x[r][k];
                     }
                 }
             }
@@ -794,9 +818,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_patches_regular(BatchArgs a)
 #pragma unroll
             for (int o = 0; o < 3; ++o)
 #pragma unroll
-                for (int q = 0; q < FC; ++q)
+                for (int f = 0; f < FC; ++f)
 #pragma unroll
-                    for (int k = 0; k < LC; ++k) acc[o][q][k] = 0.0f;
+                    for (int k = 0; k < LC; ++k) acc[o][f][k] = 0.0f;
             // the curves' values pass through an empty asm each chunk, so the
             // 48 weight products are formed per chunk instead of being held
             // in registers across the frame loop (they are the same products)
@@ -812,37 +836,39 @@ __global__ __launch_bounds__(kBlock) void k_batch_patches_regular(BatchArgs a)
                 asm volatile("" : "+v"(cb[r]), "+v"(cd[r]), "+v"(tbv[r]), "+v"(tdv[r]), "+v"(swv[r]));
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {                 // point j = 4 r + q, in order
+            for (int r = 0; r < 4; ++r) {                 // point j = 4 r + qq, in order
                 const float tb = tbv[r], td = tdv[r];
 #pragma unroll
                 for (int qq = 0; qq < 4; ++qq) {
-                    const int slot = (int)((swv[r] >> (8 * qq)) & 0xffu);
                     const float wp = cb[qq] * tb, wu = cd[qq] * tb, wvv = cb[qq] * td;
+                    const float *ps = area + ((swv[r] >> (8 * qq)) & 0xffu) * STR;
                     // every frame of the chunk without branches, so the point's
                     // LDS reads issue together (frames past the end are not stored)
-                    float x[FC][LC];
+                    float x[4 * A::NQ];
 #pragma unroll
-                    for (int q = 0; q < FC; ++q)
+                    for (int g = 0; g < A::NQ; ++g) {
+                        const v4f v = *(const v4f *)(ps + 4 * g);
 #pragma unroll
-                        for (int k = 0; k < LC; ++k) x[q][k] = Ls[q * LC + k][slot];
+                        for (int k = 0; k < 4; ++k) x[4 * g + k] = v[k];
+                    }
 #pragma unroll
-                    for (int q = 0; q < FC; ++q)
+                    for (int f = 0; f < FC; ++f)
 #pragma unroll
                         for (int k = 0; k < LC; ++k) {
-                            acc[0][q][k] += x[q][k] * wp;
-                            acc[1][q][k] += x[q][k] * wu;
-                            acc[2][q][k] += x[q][k] * wvv;
+                            acc[0][f][k] += x[f * LC + k] * wp;
+                            acc[1][f][k] += x[f * LC + k] * wu;
+                            acc[2][f][k] += x[f * LC + k] * wvv;
                         }
                     // one point's reads in flight: the point's sums are taken
                     // as asm inputs before a memory clobber, so its products
                     // are formed before the next point's LDS reads issue
-                    // (otherwise every point's 7 * FC values are held at once)
+                    // (otherwise every point's values are held at once)
 #pragma unroll
                     for (int o = 0; o < 3; ++o)
 #pragma unroll
-                        for (int q = 0; q < FC; ++q)
+                        for (int f = 0; f < FC; ++f)
 #pragma unroll
-                            for (int k = 0; k < LC; ++k) asm volatile("" ::"v"(acc[o][q][k]));
+                            for (int k = 0; k < LC; ++k) asm volatile("" ::"v"(acc[o][f][k]));
                     asm volatile("" ::: "memory");
                 }
             }
@@ -888,8 +914,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_patches(BatchArgs a)
 #pragma unroll
         for (int j = 0; j < 20; ++j) cv[j] = j < n ? max(cvs[j], 0) : 0;
 
-        for (int f0 = 0; f0 < sg.frames; f0 += FC) {
-            const int nq = min(FC, sg.frames - f0);
+        const int fEnd = item.f0 + min(a.itemFrames, sg.frames - item.f0);
+        for (int f0 = item.f0; f0 < fEnd; f0 += FC) {
+            const int nq = min(FC, fEnd - f0);
             float acc[3][FC][LC];
 #pragma unroll
             for (int o = 0; o < 3; ++o)
