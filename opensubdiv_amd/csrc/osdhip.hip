@@ -1068,31 +1068,42 @@ int osdhip_tess_coords(int scheme, int faceSize, int numRates, const int *rates,
             return OSDHIP_ERR_ARGS;
         if ((long long)t.count * numFaces > 0x7fffffffLL) return OSDHIP_ERR_ARGS;
         hipStream_t st = (hipStream_t)stream;
+        osdhip::TessPatternArgs p;
+        osdhip::TessRunArgs &a = p.a;
+        a.runs = nullptr;
+        a.numRuns = (int)t.runs.size();
+        a.perFace = t.count;
+        a.numFaces = numFaces;
+        a.uv = uv;
+        a.q.map.nodes = toCoords ? map->nodes : nullptr;
+        a.q.map.handles = toCoords ? map->handles : nullptr;
+        a.q.map.minFace = toCoords ? map->minFace : 0;
+        a.q.map.maxFace = toCoords ? map->maxFace : -1;
+        a.q.map.maxDepth = toCoords ? map->maxDepth : 0;
+        a.q.map.n = 0;
+        a.q.map.ptex = nullptr;
+        a.q.map.u = a.q.map.v = nullptr;
+        a.q.map.coords = coords;
+        a.q.faces = faces;
+        a.q.faceSizes = faceSizes;
+        a.q.ptexBase = ptexBase;
+        a.q.numFaces = numBaseFaces;
+        if (a.numRuns <= osdhip::kTessRuns && a.perFace <= osdhip::kTessPoints) {
+            std::copy(t.runs.begin(), t.runs.end(), p.runs);
+            std::fill(p.runs + a.numRuns, p.runs + osdhip::kTessRuns, osdhip::TessRun{});
+            p.blockFaces = std::max(1, osdhip::kTessBlockPoints / a.perFace);
+            const int grid = (numFaces + p.blockFaces - 1) / p.blockFaces;
+            hipLaunchKernelGGL(osdhip::k_tess_pattern, dim3(grid), dim3(kBlock),
+                               2 * sizeof(float) * (size_t)a.perFace, st, p);
+            return last_error();
+        }
         osdhip::TessRun *druns = nullptr;
         const size_t bytes = t.runs.size() * sizeof(osdhip::TessRun);
         if (hipMallocAsync((void **)&druns, bytes, st) != hipSuccess) return last_error();
         // pageable source: the copy has read it when the call returns
         hipError_t e = hipMemcpyAsync(druns, t.runs.data(), bytes, hipMemcpyHostToDevice, st);
         if (e == hipSuccess) {
-            osdhip::TessRunArgs a;
             a.runs = druns;
-            a.numRuns = (int)t.runs.size();
-            a.perFace = t.count;
-            a.numFaces = numFaces;
-            a.uv = uv;
-            a.q.map.nodes = toCoords ? map->nodes : nullptr;
-            a.q.map.handles = toCoords ? map->handles : nullptr;
-            a.q.map.minFace = toCoords ? map->minFace : 0;
-            a.q.map.maxFace = toCoords ? map->maxFace : -1;
-            a.q.map.maxDepth = toCoords ? map->maxDepth : 0;
-            a.q.map.n = 0;
-            a.q.map.ptex = nullptr;
-            a.q.map.u = a.q.map.v = nullptr;
-            a.q.map.coords = coords;
-            a.q.faces = faces;
-            a.q.faceSizes = faceSizes;
-            a.q.ptexBase = ptexBase;
-            a.q.numFaces = numBaseFaces;
             const long long threads = (long long)numFaces * a.numRuns;
             const int grid = (int)((threads + kBlock - 1) / kBlock);
             hipLaunchKernelGGL(osdhip::k_tess_runs, dim3(grid), dim3(kBlock), 0, st, a);

@@ -9,8 +9,8 @@
 // points (corners of sub-face rings, centres).  The host builds the run
 // list of a (parameterization, rates) pattern once, computing each run's
 // start and step with the reference's float expressions in the same order;
-// the kernel then emits the runs of many faces, one thread per (face, run),
-// accumulating sequentially, so every coordinate is the reference's float.
+// the kernels accumulate each run sequentially, so every coordinate is the
+// reference's float.
 #pragma once
 #include <algorithm>
 #include <cmath>
@@ -25,7 +25,6 @@ struct TessRun {
     float u, v, du, dv;      // start and step; du / dv 0 when not accumulated
     int n;                   // points
     int offset;              // first point within the face's pattern
-    int pad[2];
 };
 
 // A parameterization (bfr/parameterization.cpp:45-90): type 0 quad, 1
@@ -84,7 +83,6 @@ private:
         r.dv = dv;
         r.n = n;
         r.offset = count;
-        r.pad[0] = r.pad[1] = 0;
         runs.push_back(r);
         count += n;
     }
@@ -258,8 +256,55 @@ struct TessRunArgs {
     FaceQueryArgs q;                 // q.faces: the base face of each pattern
 };
 
-// One thread per (face, run): the run's points accumulate their step in
-// float, point by point, as the reference's iso-lines do.
+// Patterns of up to kTessPoints points and kTessRuns runs, which come with
+// the launch: a block forms the pattern once in LDS, one thread per run, then
+// its threads take the points of its faces side by side, so that the
+// coordinates are written in order.  9,600 faces x 100 points to PatchCoords
+// (19 MB): 12.9 us, bound by the chain of lookups to a point's patch (blocks
+// of 256 points 16.9 us, of 1,024 15.6 us); one thread per (face, run), each
+// writing its own run, took 22.7 us and a copy of the runs from the host.
+constexpr int kTessPoints = 4096, kTessRuns = 128;
+constexpr int kTessBlockPoints = 512;   // a block's faces hold about so many points
+
+struct TessPatternArgs {
+    TessRunArgs a;
+    int blockFaces;
+    TessRun runs[kTessRuns];
+};
+
+__global__ __launch_bounds__(kBlock) void k_tess_pattern(TessPatternArgs t)
+{
+    extern __shared__ float pat[];                    // perFace (u, v) pairs
+    const TessRunArgs &a = t.a;
+    if ((int)threadIdx.x < a.numRuns) {
+        const TessRun run = t.runs[threadIdx.x];
+        const bool accU = run.du != 0.0f, accV = run.dv != 0.0f;
+        float u = run.u, v = run.v;
+        for (int i = 0; i < run.n; ++i) {
+            pat[2 * (run.offset + i)] = u;
+            pat[2 * (run.offset + i) + 1] = v;
+            if (accU) u += run.du;
+            if (accV) v += run.dv;
+        }
+    }
+    __syncthreads();
+    const int f0 = (int)blockIdx.x * t.blockFaces;
+    const int n = min(t.blockFaces, a.numFaces - f0) * a.perFace;
+    const size_t base = (size_t)f0 * a.perFace;
+    for (int i = (int)threadIdx.x; i < n; i += kBlock) {
+        const int f = i / a.perFace, k = i - f * a.perFace;
+        const float u = pat[2 * k], v = pat[2 * k + 1];
+        if (a.uv) {
+            a.uv[2 * (base + i)] = u;
+            a.uv[2 * (base + i) + 1] = v;
+        }
+        if (a.q.map.nodes)
+            a.q.map.coords[base + i] = face_query(a.q, a.q.faces[f0 + f], (double)u, (double)v);
+    }
+}
+
+// Larger patterns, one thread per (face, run): the run's points accumulate
+// their step in float, point by point, as the reference's iso-lines do.
 __global__ __launch_bounds__(kBlock) void k_tess_runs(TessRunArgs a)
 {
     const long long idx = (long long)blockIdx.x * kBlock + threadIdx.x;
