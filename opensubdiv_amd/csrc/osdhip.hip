@@ -179,19 +179,32 @@ static int eval_csr(const float *src, osdhip_buffer_desc sd, float *const *outs,
     return OSDHIP_OK;
 }
 
-template <bool D1, bool D2>
-static void launch_patches(int lc, const PatchArgs &a, hipStream_t st)
+// order: the binned coords' numbers (evaluated by k_patches_sorted), or NULL
+// for the caller's order.
+template <bool D1, bool D2, int LC>
+static void launch_patches_lc(const PatchArgs &a, const int *order, hipStream_t st)
 {
-    const int grid = (a.n + kBlock - 1) / kBlock;
+    if (order)
+        hipLaunchKernelGGL((k_patches_sorted<D1, D2, LC>),
+                           dim3(grid_for_blocks((int)(((long long)a.n + kBlock - 1) / kBlock))),
+                           dim3(kBlock), 0, st, a, order);
+    else
+        hipLaunchKernelGGL((k_patches<D1, D2, LC>), dim3((int)(((long long)a.n + kBlock - 1) / kBlock)),
+                           dim3(kBlock), 0, st, a);
+}
+
+template <bool D1, bool D2>
+static void launch_patches(int lc, const PatchArgs &a, const int *order, hipStream_t st)
+{
     switch (lc) {
-    case 1: hipLaunchKernelGGL((k_patches<D1, D2, 1>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((k_patches<D1, D2, 2>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 3: hipLaunchKernelGGL((k_patches<D1, D2, 3>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((k_patches<D1, D2, 4>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 5: hipLaunchKernelGGL((k_patches<D1, D2, 5>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 6: hipLaunchKernelGGL((k_patches<D1, D2, 6>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    case 7: hipLaunchKernelGGL((k_patches<D1, D2, 7>), dim3(grid), dim3(kBlock), 0, st, a); break;
-    default: hipLaunchKernelGGL((k_patches<D1, D2, 8>), dim3(grid), dim3(kBlock), 0, st, a); break;
+    case 1: launch_patches_lc<D1, D2, 1>(a, order, st); break;
+    case 2: launch_patches_lc<D1, D2, 2>(a, order, st); break;
+    case 3: launch_patches_lc<D1, D2, 3>(a, order, st); break;
+    case 4: launch_patches_lc<D1, D2, 4>(a, order, st); break;
+    case 5: launch_patches_lc<D1, D2, 5>(a, order, st); break;
+    case 6: launch_patches_lc<D1, D2, 6>(a, order, st); break;
+    case 7: launch_patches_lc<D1, D2, 7>(a, order, st); break;
+    default: launch_patches_lc<D1, D2, 8>(a, order, st); break;
     }
 }
 
@@ -790,9 +803,10 @@ static int eval_patches(const float *src, osdhip_buffer_desc srcDesc, float *con
     hipStream_t st = (hipStream_t)stream;
 
     // Patch-ordered evaluation: the coords binned by patch (patch_sort.h) in
-    // stream-ordered scratch memory, then evaluation in that order.
-    // Outputs still go to each coord's own row.
+    // stream-ordered scratch memory, then ordered by patch where they are
+    // evaluated.  Outputs still go to each coord's own row.
     void *owned = nullptr;
+    const int *sorted = nullptr;
     if (order == PatchOrder::SortedMalloc) {
         if (hipMallocAsync(&owned, PatchSortLayout(numPatchCoords).bytes, st) == hipSuccess) {
             ws = (char *)owned;
@@ -803,7 +817,7 @@ static int eval_patches(const float *src, osdhip_buffer_desc srcDesc, float *con
         }
     }
     if (order != PatchOrder::Caller && ws) {
-        a.order = queue_patch_sort(coords, numPatchCoords, ws, st);
+        sorted = queue_patch_sort(coords, numPatchCoords, ws, st);
         int rc = last_error();
         if (rc != OSDHIP_OK) {
             if (owned) (void)hipFreeAsync(owned, st);
@@ -818,9 +832,9 @@ static int eval_patches(const float *src, osdhip_buffer_desc srcDesc, float *con
             a.dst[o] = outs[o] ? outs[o] + ods[o].offset + e0 : nullptr;
             a.dstStride[o] = outs[o] ? ods[o].stride : 0;
         }
-        if (d2) launch_patches<true, true>(lc, a, st);
-        else if (d1) launch_patches<true, false>(lc, a, st);
-        else launch_patches<false, false>(lc, a, st);
+        if (d2) launch_patches<true, true>(lc, a, sorted, st);
+        else if (d1) launch_patches<true, false>(lc, a, sorted, st);
+        else launch_patches<false, false>(lc, a, sorted, st);
         rc = last_error();
     }
     if (owned) {

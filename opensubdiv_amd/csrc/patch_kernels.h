@@ -21,7 +21,6 @@ struct PatchArgs {
     const osdhip_patch_array *arrays;
     const int *indices;
     const osdhip_patch_param *params;
-    const int *order;       // evaluation order (coord index per lane), NULL = identity
 };
 
 // acc[o][k] += v[k] * weight_o[j], in the reference's point order.
@@ -76,17 +75,11 @@ __device__ __forceinline__ void gather_points(const float *src, size_t sstride, 
     }
 }
 
+// Evaluates coord c and writes its results to row i of the outputs.
 template <bool D1, bool D2, int LC>
-__global__ __launch_bounds__(kBlock) void k_patches(PatchArgs a)
+__device__ __forceinline__ void eval_patch_coord(const PatchArgs &a, const osdhip_patch_coord &c,
+                                                 int i)
 {
-    const int lane_i = (int)(blockIdx.x * kBlock + threadIdx.x);
-    if (lane_i >= a.n) return;
-    // Each coord's result depends on that coord only, so any order gives the
-    // same bits; a patch-sorted order makes neighbouring lanes share control
-    // points and index rows in L2.
-    const int i = a.order ? a.order[lane_i] : lane_i;
-
-    const osdhip_patch_coord c = a.coords[i];
     const osdhip_patch_array arr = a.arrays[c.arrayIndex];
     const osdhip_patch_param pp = a.params[c.patchIndex];
     const unsigned f1 = pp.field1;
@@ -175,6 +168,14 @@ __global__ __launch_bounds__(kBlock) void k_patches(PatchArgs a)
 #pragma unroll
         for (int k = 0; k < LC; ++k) d[k] = acc[o][k] * f;
     }
+}
+
+template <bool D1, bool D2, int LC>
+__global__ __launch_bounds__(kBlock) void k_patches(PatchArgs a)
+{
+    const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
+    if (i >= a.n) return;
+    eval_patch_coord<D1, D2, LC>(a, a.coords[i], i);
 }
 
 // Limit normals from EvalPatches' first derivatives, one thread per point:
