@@ -47,6 +47,11 @@ class BatchStencils(C.Structure):
                 ("frames", C.c_int), ("stage", C.c_int)]
 
 
+class UploadBlock(C.Structure):
+    """osdhip_upload_block."""
+    _fields_ = [("dst", C.c_void_p), ("src", C.c_void_p), ("bytes", C.c_longlong)]
+
+
 class BatchPatches(C.Structure):
     """osdhip_batch_patches."""
     _fields_ = [("numCoords", C.c_int), ("coords", C.c_void_p), ("arrays", C.c_void_p),
@@ -116,6 +121,7 @@ _HIP_SIGS = {
     "osdhip_batch_patch_staging": [_vp, _i, _vp, _vp, _vp, _vp, _vp],
     "osdhip_batch_epoch_bytes": [_i, _i, _vp, _i, _vp, _i],
     "osdhip_batch_epoch": [_i, _i, _vp, _i, _vp, _i, _vp, C.c_longlong, _vp, C.c_longlong, _vp],
+    "osdhip_batch_upload": [_i, _vp, _vp],
 }
 
 _hip = None

@@ -991,4 +991,48 @@ int osdhip_batch_epoch(int length, int numStencilSegments, const osdhip_batch_st
     return OSDHIP_OK;
 }
 
+int osdhip_batch_upload(int n, const osdhip_upload_block *blocks, void *stream)
+{
+    if (n < 0 || (n > 0 && !blocks)) return OSDHIP_ERR_ARGS;
+    for (int i = 0; i < n; ++i) {
+        const osdhip_upload_block &b = blocks[i];
+        if (b.bytes < 0 || (b.bytes & 3) || ((size_t)b.dst & 3) || ((size_t)b.src & 3) ||
+            b.bytes / kUploadBlock > INT_MAX / (2 * kUploadBlocks))
+            return OSDHIP_ERR_ARGS;
+        if (b.bytes == 0) continue;
+        // both ends of the source, the start of the destination
+        const char *ends[3] = { (const char *)b.src, (const char *)b.src + b.bytes - 4,
+                                (const char *)b.dst };
+        for (int k = 0; k < 3; ++k) {
+            hipPointerAttribute_t at;
+            if (hipPointerGetAttributes(&at, ends[k]) != hipSuccess) {
+                (void)hipGetLastError();
+                return OSDHIP_ERR_ARGS;
+            }
+            if (at.type != (k < 2 ? hipMemoryTypeHost : hipMemoryTypeDevice) ||
+                (const char *)at.devicePointer != ends[k])
+                return OSDHIP_ERR_ARGS;
+        }
+    }
+    for (int i = 0; i < n;) {
+        UploadArgs a;
+        std::memset(&a, 0, sizeof(a));
+        for (; i < n && a.n < kUploadBlocks; ++i) {
+            if (blocks[i].bytes == 0) continue;
+            a.dst[a.n] = (int *)blocks[i].dst;
+            a.src[a.n] = (const int *)blocks[i].src;
+            a.words[a.n] = blocks[i].bytes / 4;
+            a.end[a.n] = (a.n ? a.end[a.n - 1] : 0) +
+                         (int)((blocks[i].bytes + kUploadBlock - 1) / kUploadBlock);
+            ++a.n;
+        }
+        if (a.n == 0) break;
+        hipLaunchKernelGGL(k_batch_upload, dim3(a.end[a.n - 1]), dim3(kBlock), 0,
+                           (hipStream_t)stream, a);
+        int rc = last_error();
+        if (rc != OSDHIP_OK) return rc;
+    }
+    return OSDHIP_OK;
+}
+
 }  // extern "C"

@@ -963,4 +963,48 @@ __global__ __launch_bounds__(kBlock) void k_batch_patches(BatchArgs a)
     }
 }
 
+// Frame uploads of an epoch (osdhip_batch_upload): the kernel reads the pinned
+// frames over the host link itself.  A block of threads copies kUploadBlock
+// bytes, all its loads in flight before the first store.  Bound by the link;
+// what it saves is a copy command, with its own start and completion, per
+// frame (an epoch of 10 requests: 162 -> 115 us a call, most of it spent
+// queueing).
+constexpr int kUploadBlocks = 32;               // host blocks per launch
+constexpr int kUploadLoads = 2;                 // 16-byte loads per thread
+constexpr long long kUploadBlock = 16LL * kUploadLoads * kBlock;
+struct UploadArgs {
+    int n;
+    int end[kUploadBlocks];                     // first grid block past each host block
+    int *dst[kUploadBlocks];
+    const int *src[kUploadBlocks];
+    long long words[kUploadBlocks];
+};
+typedef int v4i_word __attribute__((ext_vector_type(4), aligned(4)));
+__global__ __launch_bounds__(kBlock) void k_batch_upload(UploadArgs a)
+{
+    const int b = (int)blockIdx.x;
+    int s = 0;
+    while (s < a.n - 1 && b >= a.end[s]) ++s;
+    const long long first = (long long)(b - (s ? a.end[s - 1] : 0)) * (kUploadBlock / 4);
+    const int *src = a.src[s] + first;
+    int *dst = a.dst[s] + first;
+    const long long left = a.words[s] - first;  // >= 1
+    const int t = 4 * (int)threadIdx.x;
+    if (left >= kUploadBlock / 4) {
+        v4i_word v[kUploadLoads];
+#pragma unroll
+        for (int k = 0; k < kUploadLoads; ++k)
+            v[k] = *(const v4i_word *)(src + t + 4 * kBlock * k);
+#pragma unroll
+        for (int k = 0; k < kUploadLoads; ++k) *(v4i_word *)(dst + t + 4 * kBlock * k) = v[k];
+        return;
+    }
+    const int m = (int)left;
+    const int whole = m & ~3;
+    for (int j = t; j < whole; j += 4 * kBlock)
+        *(v4i_word *)(dst + j) = *(const v4i_word *)(src + j);
+    const int j = whole + (int)threadIdx.x;
+    if (j < m) dst[j] = src[j];
+}
+
 }  // namespace osdhip

@@ -2,11 +2,14 @@
 // and the C ABI declared in include/osdhip.h.
 //
 // Stencil evaluation is a sparse gather (CSR rows x a dense multi-column
-// source), HBM-bound at < 0.3 FLOP/byte, so it uses no MFMA.  Two kernels:
-//   * stencil_csr.h    - raw Far CSR tables (the raw EvalStencils entry
-//                        points): per-wave LDS staging of the table slice;
-//   * stencil_sliced.h - HipStencilTable's device layout (64-row column-major
-//                        slices): coalesced streaming without LDS.
+// source), HBM-bound at < 0.3 FLOP/byte, so it uses no MFMA.  Three kernels:
+//   * stencil_csr.h     - raw Far CSR tables (the raw EvalStencils entry
+//                         points): per-wave LDS staging of the table slice;
+//   * stencil_compact.h - HipStencilTable's compact slices (layouts 0 and 2):
+//                         control vertices listed per 64-row slice, staged in
+//                         LDS, named by one byte per entry;
+//   * stencil_sliced.h  - 64-row column-major slices (layouts 1 and 3):
+//                         coalesced streaming without LDS.
 // All weight arrays of a derivative table (P, du, dv [, duu, duv, dvv])
 // share the index stream and are applied in ONE launch.
 //

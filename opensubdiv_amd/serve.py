@@ -151,8 +151,13 @@ class Server:
         self.copying = []                        # requests whose results are downloading
         self.inflight = []                       # (event, request) per chunk, in issue order
         # host frames in pinned memory, one block per topology
-        self.frames = [torch.from_numpy(np.ascontiguousarray(r.frames)).pin_memory()
+        self.frames = [torch.from_numpy(np.ascontiguousarray(r.frames, np.float32)).pin_memory()
                        for r in residents]
+
+    def __del__(self):
+        # epochs in flight read the pinned frames and write the arenas
+        for slot in getattr(self, "slots", []):
+            slot["event"].synchronize()
 
     # ---- sizes ----------------------------------------------------------
     def dev_floats(self, r: Request):
@@ -227,12 +232,20 @@ class Server:
             slot["scratch"] = torch.empty(cap, dtype=torch.uint8, device="cuda")
             slot["cap"] = cap
         st = slot["stream"]
+        base, ups = self.dev.data_ptr(), []
+        for r in reqs:
+            f = self.frames[r.topo]
+            n = self.res[r.topo].nctrl * self.L
+            if f.numel() != f.shape[0] * n:
+                raise RuntimeError(f"topology {r.topo}: frames of {f.numel() // f.shape[0]} "
+                                   f"values, {n} expected")
+            ups.append(_lib.UploadBlock(base + 4 * r.dev[0][0],
+                                        f.data_ptr() + 4 * n * (r.frame % f.shape[0]), 4 * n))
         with torch.cuda.stream(st):
-            for r in reqs:
-                t = self.res[r.topo]
-                src = self.frames[r.topo][r.frame % self.frames[r.topo].shape[0]].reshape(-1)
-                o, _ = r.dev[0]
-                self.dev[o:o + t.nctrl * self.L].copy_(src, non_blocking=True)
+            rc = self.lib.osdhip_batch_upload(
+                len(ups), ctypes.cast((_lib.UploadBlock * max(1, len(ups)))(*ups),
+                                      ctypes.c_void_p), st.cuda_stream)
+            _lib.check(rc, "osdhip_batch_upload")
             rc = self.lib.osdhip_batch_epoch(self.L, nS, ctypes.cast(SA, ctypes.c_void_p), nP,
                                              ctypes.cast(PA, ctypes.c_void_p), self.item_slices,
                                              slot["staging"].data_ptr(), slot["cap"],
