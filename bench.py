@@ -489,7 +489,8 @@ def run_patches(args, lib, inputs, with_cpu):
            "gregory_patches": int(sum(a["numPatches"] for a in pt.arrays if a["desc"] == 9)),
            "algorithmic_bytes": alg, "GBps": alg / (avg * 1e-3) / 1e9,
            "frac_of_peak": alg / (avg * 1e-3) / 1e9 / HBM_PEAK_GBS,
-           "kernel": f"k_patches<true,false,3> ({best})", "autotune": variants}
+           "kernel": ("k_patches_sorted<true,false,3>" if best == "patch_sorted"
+                      else "k_patches<true,false,3>") + f" ({best})", "autotune": variants}
     got = [o.cpu().numpy().reshape(n, L) for o in outs]
     if inputs.get("points64") is not None:
         import oracle
