@@ -508,8 +508,9 @@ int osdhip_batch_epoch(int length, int numStencilSegments, const osdhip_batch_st
 /* Frame uploads of an epoch: copies n blocks of pinned host memory
  * (hipHostMalloc) to device memory on `stream`, one kernel launch per 32
  * blocks.  Addresses and sizes are multiples of 4 bytes; a block whose source
- * is not pinned host memory or whose destination is not device memory is
- * OSDHIP_ERR_ARGS, before anything is queued.  The blocks must not overlap and
+ * is not pinned host memory, or whose destination is not memory of the current
+ * device, from its first byte to its last is OSDHIP_ERR_ARGS, before anything
+ * is queued.  The blocks must not overlap and
  * must stay as they are until the work queued on `stream` has completed. */
 typedef struct {
     void *dst;

@@ -991,28 +991,73 @@ int osdhip_batch_epoch(int length, int numStencilSegments, const osdhip_batch_st
     return OSDHIP_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The allocations one osdhip_batch_upload call has looked up: its blocks
+// mostly lie in one arena and a few frame pools, each then looked up once.
+class KnownMemory {
+    struct Range {
+        const char *lo, *hi;
+        bool host;
+    };
+    Range r[8];
+    int n = 0, device = -1;
+
+    // The allocation holding p, pinned host memory or memory of the current
+    // device; NULL when p is in neither.
+    const Range *find(const char *p, bool host)
+    {
+        for (int k = 0; k < std::min(n, 8); ++k)
+            if (r[k].host == host && p >= r[k].lo && p < r[k].hi) return &r[k];
+        hipPointerAttribute_t at;
+        void *base = nullptr;
+        size_t size = 0;
+        if ((device < 0 && hipGetDevice(&device) != hipSuccess) ||
+            hipPointerGetAttributes(&at, p) != hipSuccess ||
+            at.type != (host ? hipMemoryTypeHost : hipMemoryTypeDevice) ||
+            (const char *)at.devicePointer != p || (!host && at.device != device) ||
+            hipMemGetAddressRange((hipDeviceptr_t *)&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        Range &f = r[n++ % 8];
+        f = { (const char *)base, (const char *)base + size, host };
+        return p >= f.lo && p < f.hi ? &f : nullptr;
+    }
+
+public:
+    // Whether all of [p, p + bytes) is such memory (adjacent allocations may
+    // share it); bytes > 0.
+    bool covers(const void *p, long long bytes, bool host)
+    {
+        const char *at = (const char *)p, *end = at + bytes;
+        while (at < end) {
+            const Range *f = find(at, host);
+            if (!f) return false;
+            at = f->hi;
+        }
+        return true;
+    }
+};
+
+}  // namespace
+
+extern "C" {
+
 int osdhip_batch_upload(int n, const osdhip_upload_block *blocks, void *stream)
 {
     if (n < 0 || (n > 0 && !blocks)) return OSDHIP_ERR_ARGS;
+    KnownMemory known;
     for (int i = 0; i < n; ++i) {
         const osdhip_upload_block &b = blocks[i];
         if (b.bytes < 0 || (b.bytes & 3) || ((size_t)b.dst & 3) || ((size_t)b.src & 3) ||
             b.bytes / kUploadBlock > INT_MAX / (2 * kUploadBlocks))
             return OSDHIP_ERR_ARGS;
         if (b.bytes == 0) continue;
-        // both ends of the source, the start of the destination
-        const char *ends[3] = { (const char *)b.src, (const char *)b.src + b.bytes - 4,
-                                (const char *)b.dst };
-        for (int k = 0; k < 3; ++k) {
-            hipPointerAttribute_t at;
-            if (hipPointerGetAttributes(&at, ends[k]) != hipSuccess) {
-                (void)hipGetLastError();
-                return OSDHIP_ERR_ARGS;
-            }
-            if (at.type != (k < 2 ? hipMemoryTypeHost : hipMemoryTypeDevice) ||
-                (const char *)at.devicePointer != ends[k])
-                return OSDHIP_ERR_ARGS;
-        }
+        if (!known.covers(b.src, b.bytes, true) || !known.covers(b.dst, b.bytes, false))
+            return OSDHIP_ERR_ARGS;
     }
     for (int i = 0; i < n;) {
         UploadArgs a;

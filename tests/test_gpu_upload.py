@@ -51,3 +51,28 @@ def test_refused_pointers_and_sizes(hip):
             _lib.ERR_ARGS, bad
     torch.cuda.synchronize()
     assert bool((dst == 1).all())
+
+
+def test_blocks_that_run_past_their_allocation_are_refused(hip):
+    """A block whose destination (or source) starts in an allocation and ends
+    past it is refused, and so is everything given beside it; one that ends
+    with the allocation is copied."""
+    src = torch.arange(64, dtype=torch.int32).pin_memory()        # 256 bytes
+    more = torch.zeros(1024, dtype=torch.int32).pin_memory()
+    dst = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    short = ctypes.c_void_p()
+    assert hip.osdhip_malloc(ctypes.byref(short), 256) == 0
+    try:
+        for bad in ((short.value, more.data_ptr(), 260), (short.value + 128, more.data_ptr(), 256),
+                    (short.value, more.data_ptr(), 4096), (dst.data_ptr(), src.data_ptr(), 260)):
+            assert upload(hip, [_lib.UploadBlock(dst.data_ptr(), src.data_ptr(), 256),
+                                _lib.UploadBlock(*bad)]) == _lib.ERR_ARGS, bad
+        torch.cuda.synchronize()
+        assert bool((dst == 0).all())
+        assert upload(hip, [_lib.UploadBlock(short.value, src.data_ptr(), 256)]) == 0
+        got = np.zeros(64, np.int32)
+        assert hip.osdhip_memcpy_dtoh(got.ctypes.data, short, 256, stream()) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(got, np.arange(64))
+    finally:
+        hip.osdhip_free(short)
