@@ -241,18 +241,24 @@ class Server:
                                    f"values, {n} expected")
             ups.append(_lib.UploadBlock(base + 4 * r.dev[0][0],
                                         f.data_ptr() + 4 * n * (r.frame % f.shape[0]), 4 * n))
-        with torch.cuda.stream(st):
-            rc = self.lib.osdhip_batch_upload(
-                len(ups), ctypes.cast((_lib.UploadBlock * max(1, len(ups)))(*ups),
-                                      ctypes.c_void_p), st.cuda_stream)
-            _lib.check(rc, "osdhip_batch_upload")
-            rc = self.lib.osdhip_batch_epoch(self.L, nS, ctypes.cast(SA, ctypes.c_void_p), nP,
-                                             ctypes.cast(PA, ctypes.c_void_p), self.item_slices,
-                                             slot["staging"].data_ptr(), slot["cap"],
-                                             slot["scratch"].data_ptr(), slot["cap"],
-                                             st.cuda_stream)
-            _lib.check(rc, "osdhip_batch_epoch")
-            slot["event"].record(st)
+        try:
+            with torch.cuda.stream(st):
+                rc = self.lib.osdhip_batch_upload(
+                    len(ups), ctypes.cast((_lib.UploadBlock * max(1, len(ups)))(*ups),
+                                          ctypes.c_void_p), st.cuda_stream)
+                _lib.check(rc, "osdhip_batch_upload")
+                rc = self.lib.osdhip_batch_epoch(self.L, nS, ctypes.cast(SA, ctypes.c_void_p), nP,
+                                                 ctypes.cast(PA, ctypes.c_void_p), self.item_slices,
+                                                 slot["staging"].data_ptr(), slot["cap"],
+                                                 slot["scratch"].data_ptr(), slot["cap"],
+                                                 st.cuda_stream)
+                _lib.check(rc, "osdhip_batch_epoch")
+                slot["event"].record(st)
+        except BaseException:
+            # what got queued reads the pinned frames and the staging block and
+            # writes the arena, and no event will tell when it is done
+            st.synchronize()
+            raise
         slot["reqs"] = reqs
         self.epochs.append(len(reqs))
         self.epoch_points.append(sum(self.points(r) for r in reqs))
