@@ -68,16 +68,24 @@ struct EntryGroup {
     float w[NWT][4];
 };
 
+// Reads *p; STREAM: data the call reads once.
+template <bool STREAM, class P>
+__device__ __forceinline__ auto load_entry(P p)
+{
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
 // Loads group g of a slice's weights: wp = the slice's weights (wave-uniform);
 // 4 g < W.  Columns past W get weight 0.
-template <int NWT, class P>
+template <int NWT, bool STREAM = true, class P>
 __device__ __forceinline__ void load_weights(P wp, int W, int g, int lane, float (&w)[NWT][4])
 {
     const int left = W - 4 * g;                        // wave-uniform
     if constexpr (NWT == 1) {
         P p = wp + (size_t)g * (4 * kWave);
         if (left >= 4) {
-            const v4f q = __builtin_nontemporal_load((const OSDHIP_GLOBAL v4f *)(p + 4 * lane));
+            const v4f q = load_entry<STREAM>((const OSDHIP_GLOBAL v4f *)(p + 4 * lane));
 #pragma unroll
             for (int u = 0; u < 4; ++u) w[0][u] = q[u];
         } else {
@@ -95,7 +103,7 @@ __device__ __forceinline__ void load_weights(P wp, int W, int g, int lane, float
             // past the width: the last column again, with weight 0
             P q = p + (size_t)min(u, left - 1) * (NWT * kWave);
 #pragma unroll
-            for (int k = 0; k < NWT; ++k) w[k][u] = __builtin_nontemporal_load(q + k);
+            for (int k = 0; k < NWT; ++k) w[k][u] = load_entry<STREAM>(q + k);
         }
 #pragma unroll
         for (int u = 1; u < 4; ++u)

@@ -121,6 +121,63 @@ def test_batch_list_edges(L, frames):
             b.close()
 
 
+def ragged_table(rng, widths, nlist, nsrc=900):
+    """Slices of 64 rows (and one of 29) of up to `widths` entries, each drawn
+    from `nlist` vertices of its own (None: from all, so that the locality
+    orders list none of them)."""
+    sizes, indices = [], []
+    for s, W in enumerate(widths):
+        pool = np.arange(nsrc) if nlist is None else rng.choice(nsrc, size=nlist, replace=False)
+        for r in range(64 if s + 1 < len(widths) else 29):
+            n = 0 if r == 7 else W if r % 4 == 0 else int(rng.integers(1, W + 1))
+            sizes.append(n)
+            indices.append(rng.choice(pool, size=n, replace=False))
+    t = {"sizes": np.array(sizes, np.int32), "indices": np.concatenate(indices).astype(np.int32)}
+    t["offsets"] = (np.cumsum(t["sizes"]) - t["sizes"]).astype(np.int32)
+    t["weights"] = rng.normal(size=len(t["indices"])).astype(np.float32)
+    return t
+
+
+def batch_matches(t, layout, order, L, frames, nsrc=900):
+    """The batch kernel's variants on one table against the oracle."""
+    import torch
+    rng = np.random.default_rng(L + 16 * frames)
+    n = len(t["sizes"])
+    table = HipStencilTable.Create(t, layout=layout, order=order, keep_csr=False)
+    src = rng.normal(size=(nsrc, frames, L)).astype(np.float32)
+    s_t = dev(src)
+    want = [oracle.apply_stencils(np.ascontiguousarray(src[:, f]), t["sizes"], t["offsets"],
+                                  t["indices"], t["weights"]) for f in range(frames)]
+    for vertex_major in (False, True):
+        out = empty(n * frames * L)
+        b = Batch(L, [dict(table=table, src=s_t, src_v=frames * L, src_f=L, dst=out, frames=frames,
+                           dst_v=frames * L if vertex_major else L,
+                           dst_f=L if vertex_major else n * L)])
+        for fc in (1, 2, 4):
+            assert b.set("a_frames", fc) == 0
+            assert b.set("a_group", 2 if layout == 0 and fc == 4 else 4) == 0
+            out.fill_(float("nan"))
+            b.run(1)
+            torch.cuda.synchronize()
+            got = out.cpu().numpy()
+            got = got.reshape(n, frames, L).transpose(1, 0, 2) if vertex_major \
+                else got.reshape(frames, n, L)
+            for f in range(frames):
+                np.testing.assert_array_equal(got[f], want[f], err_msg=f"chunk {fc} frame {f}")
+        b.close()
+    return table.layout()
+
+
+@pytest.mark.parametrize("L", [1, 4, 5, 7, 8])
+@pytest.mark.parametrize("frames", [1, 2, 3, 5])
+def test_batch_unlisted_slices(L, frames):
+    """Slices without a list, of widths at and beside the entries that one
+    chunk of 1, 2 or 4 frames gathers at a time (8, 4, 2)."""
+    t = ragged_table(np.random.default_rng(L), (2, 3, 4, 5, 6, 7, 8, 9, 12, 17, 31, 8), None)
+    info = batch_matches(t, 2, 0, L, frames)
+    assert info["listed_slices"] < info["slices"] // 2
+
+
 @pytest.mark.parametrize("n,level,far_order", [(7, 4, True), (14, 3, False)])
 def test_large_order_2_tables(hip, n, level, far_order):
     """Tables of 65,536 rows and more under order 2: a level-4 refinement table
