@@ -355,7 +355,13 @@ __device__ __forceinline__ void add_entry(const float *p, float w, float (&acc)[
 }
 
 // One listed slice for every frame, FC per chunk (U <= batch_list at FC).
-// RES: the slice's entries (W <= kBatchWidth) stay in registers.
+// RES: the slice's entries (W <= kBatchWidth) stay in registers.  A wider
+// slice reads them from the caches for every chunk, four at a time, and
+// stages a chunk when it gets to it: this keeps its registers below the RES
+// path's, whose waves per SIMD it shares (eight or sixteen entries read ahead:
+// 14 to 25 VGPRs more).  1.3 M rows of 14 entries on average, slices up to 18
+// wide (valence-6 vertices), 16 frames of 7 floats: 606 us at FC = 4, 940 one
+// frame at a time.
 template <int LC, int FC, bool RES>
 __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float *area, int *rowsL,
                                                    const G_ unsigned *rp, const G_ float *wp, int W,
@@ -375,8 +381,8 @@ __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float 
 #pragma unroll
         for (int c = 0; c < GR; ++c)
             if (g0 + c < G) {                          // wave-uniform
-                e[c].slots = __builtin_nontemporal_load(rp + (size_t)(g0 + c) * kWave + lane);
-                load_weights<1>(wp, W, g0 + c, lane, e[c].w);
+                e[c].slots = load_entry<RES>(rp + (size_t)(g0 + c) * kWave + lane);
+                load_weights<1, RES>(wp, W, g0 + c, lane, e[c].w);
             }
     };
     int vtx[LISTS];
@@ -406,8 +412,9 @@ __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float 
     // through LDS so that consecutive lanes store one row's run
     const bool runs = sg.dstF == LC && sg.frames > 1;
     if (runs) rowsL[lane] = active ? row : -1;
-    stage(0);
+    if (RES) stage(0);
     for (int f0 = 0; f0 < sg.frames; f0 += FC) {
+        if (!RES) stage(f0);
         wave_lds_sync();                               // previous chunk's reads are done
 #pragma unroll
         for (int r = 0; r < kStageQuads; ++r) {
@@ -421,7 +428,7 @@ __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float 
         if (lane < A::STR) area[U * A::STR + lane] = 0.0f;   // the zero slot
         wave_lds_sync();
         // the next chunk's loads are in flight while this one is summed
-        if (f0 + FC < sg.frames) stage(f0 + FC);
+        if (RES && f0 + FC < sg.frames) stage(f0 + FC);
         float acc[FC][LC];
 #pragma unroll
         for (int f = 0; f < FC; ++f)
@@ -430,7 +437,10 @@ __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float 
         auto entries = [&](auto frames) {
             constexpr int NF = decltype(frames)::value;
             for (int g0 = 0; g0 < (RES ? 1 : G); g0 += GR) {
-                if (!RES) load(g0);
+                if (!RES) {
+                    asm volatile("" ::: "memory");     // no loads moved up here
+                    load(g0);
+                }
 #pragma unroll
                 for (int g = 0; g < GR; ++g) {
                     if (g0 + g < G) {                  // wave-uniform
@@ -572,15 +582,21 @@ __global__ __launch_bounds__(kBlock) void k_batch_stencils(BatchArgs a)
             int *rowsL = rowsLds[wv];
             // a list too long for FC frames at once takes fewer per chunk
             static_assert(batch_list<LC, 1, FLOATS>() == kSliceList, "every list fits at one frame");
-            if (W > kBatchWidth)
-                batch_listed_slice<LC, 1, false>(sg, area, rowsL, rp, wp, W, U, list, row, active);
-            else if (FC == 4 && U <= batch_list<LC, FC, FLOATS>())
-                batch_listed_slice<LC, FC, true>(sg, area, rowsL, rp, wp, W, U, list, row, active);
+            auto listed = [&](auto frames) {
+                constexpr int F = decltype(frames)::value;
+                if (W <= kBatchWidth)
+                    batch_listed_slice<LC, F, true>(sg, area, rowsL, rp, wp, W, U, list, row,
+                                                    active);
+                else
+                    batch_listed_slice<LC, F, false>(sg, area, rowsL, rp, wp, W, U, list, row,
+                                                     active);
+            };
+            if (FC == 4 && U <= batch_list<LC, FC, FLOATS>())
+                listed(std::integral_constant<int, FC>{});
             else if (FC >= 2 && U <= batch_list<LC, FC < 2 ? 1 : 2, FLOATS>())
-                batch_listed_slice<LC, FC < 2 ? 1 : 2, true>(sg, area, rowsL, rp, wp, W, U, list,
-                                                             row, active);
+                listed(std::integral_constant<int, FC < 2 ? 1 : 2>{});
             else
-                batch_listed_slice<LC, 1, true>(sg, area, rowsL, rp, wp, W, U, list, row, active);
+                listed(std::integral_constant<int, 1>{});
         }
     }
 }

@@ -178,6 +178,18 @@ def test_batch_unlisted_slices(L, frames):
     assert info["listed_slices"] < info["slices"] // 2
 
 
+@pytest.mark.parametrize("L", [1, 4, 5, 7, 8])
+@pytest.mark.parametrize("frames", [1, 2, 3, 5])
+@pytest.mark.parametrize("nlist", [40, 64, 65, 128, 250])
+def test_batch_wide_listed_slices(L, frames, nlist):
+    """Listed slices wider than the 16 entries held in registers, at every
+    remainder of the groups of four, with lists at and beside those that 4 and
+    2 frames per chunk take."""
+    t = ragged_table(np.random.default_rng(L), (16, 17, 18, 19, 20, 21, 24, 33, 40), nlist)
+    info = batch_matches(t, 0, 0, L, frames)
+    assert info["listed_slices"] == info["slices"]
+
+
 @pytest.mark.parametrize("n,level,far_order", [(7, 4, True), (14, 3, False)])
 def test_large_order_2_tables(hip, n, level, far_order):
     """Tables of 65,536 rows and more under order 2: a level-4 refinement table
