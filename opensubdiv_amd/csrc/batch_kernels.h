@@ -402,7 +402,8 @@ __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float 
 #pragma unroll
         for (int r = 0; r < kStageQuads; ++r)
             if (r * VI < U) {                          // wave-uniform
-                const int v = __shfl(vtx[r / QV], (r * VI + lane / QV) % kWave, kWave);
+                int v = vtx[r / QV];                   // one quad per vertex: the lane's own
+                if (QV > 1) v = __shfl(v, (r * VI + lane / QV) % kWave, kWave);
                 const G_ float *pv = p + (size_t)(unsigned)v * sg.srcV;
 #pragma unroll
                 for (int k = 0; k < N; ++k) x[r][k] = pv[k];
@@ -435,7 +436,12 @@ __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float 
 #pragma unroll
             for (int k = 0; k < LC; ++k) acc[f][k] = 0.0f;
         auto entries = [&](auto frames) {
-            constexpr int NF = decltype(frames)::value;
+            constexpr int NF = decltype(frames)::value, NQ = (NF * LC + 3) / 4;
+            // entries whose LDS reads are in flight together: 16 floats of
+            // them, where a batch is small enough to wait for them (221 K
+            // rows, 12 frames of 2 floats: 36.2 us one by one, 33.8 in fours);
+            // hoisting all reads would cut occupancy
+            constexpr int FLIGHT = NQ == 1 ? 4 : NQ == 2 ? 2 : 1;
             for (int g0 = 0; g0 < (RES ? 1 : G); g0 += GR) {
                 if (!RES) {
                     asm volatile("" ::: "memory");     // no loads moved up here
@@ -453,9 +459,7 @@ __device__ __forceinline__ void batch_listed_slice(const GStencilSeg &sg, float 
                         for (int u = 0; u < 4; ++u) {
                             add_entry<LC, FC, NF>(area + ((slots >> (8 * u)) & 0xffu) * A::STR,
                                                   e[g].w[0][u], acc);
-                            // one entry's LDS reads in flight at a time:
-                            // hoisting all of them would cut occupancy
-                            __builtin_amdgcn_sched_barrier(0);
+                            if ((u + 1) % FLIGHT == 0) __builtin_amdgcn_sched_barrier(0);
                         }
                     }
                 }
@@ -580,7 +584,8 @@ __global__ __launch_bounds__(kBlock) void k_batch_stencils(BatchArgs a)
             const G_ int *list = sg.ctrl + ds.ctrlOff;
             float *area = lds[wv];
             int *rowsL = rowsLds[wv];
-            // a list too long for FC frames at once takes fewer per chunk
+            // a list too long for FC frames at once takes fewer per chunk, and
+            // so does a segment of fewer frames
             static_assert(batch_list<LC, 1, FLOATS>() == kSliceList, "every list fits at one frame");
             auto listed = [&](auto frames) {
                 constexpr int F = decltype(frames)::value;
@@ -591,9 +596,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_stencils(BatchArgs a)
                     batch_listed_slice<LC, F, false>(sg, area, rowsL, rp, wp, W, U, list, row,
                                                      active);
             };
-            if (FC == 4 && U <= batch_list<LC, FC, FLOATS>())
+            if (FC == 4 && sg.frames > 2 && U <= batch_list<LC, FC, FLOATS>())
                 listed(std::integral_constant<int, FC>{});
-            else if (FC >= 2 && U <= batch_list<LC, FC < 2 ? 1 : 2, FLOATS>())
+            else if (FC >= 2 && sg.frames > 1 && U <= batch_list<LC, FC < 2 ? 1 : 2, FLOATS>())
                 listed(std::integral_constant<int, FC < 2 ? 1 : 2>{});
             else
                 listed(std::integral_constant<int, 1>{});
