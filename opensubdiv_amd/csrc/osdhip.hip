@@ -64,22 +64,32 @@ static void launch_rec_paired(int lc, int group, const RecArgs &a, int grid, hip
     else launch_rec_paired_g<8>(lc, a, grid, st);
 }
 
-template <int NWT>
-static void launch_compact(int lc, const CompactArgs &a, int grid, hipStream_t st)
+template <int NWT, int LC>
+static void launch_compact_lc(const CompactArgs &a, bool lists, int grid, hipStream_t st)
 {
+    if constexpr (NWT == 1 && LC > 4) {
+        if (!lists) {
+            hipLaunchKernelGGL((k_stencils_compact<NWT, LC, false>), dim3(grid), dim3(kBlock), 0, st, a);
+            return;
+        }
+    }
     // dynamic LDS: four waves' slots (at most 4 * 256 * 32 B)
-    const size_t lds = sizeof(float) * kWavesPerBlock * (size_t)a.slots *
-                       (lc == 1 ? SlotShape<1>::STR : lc == 2 ? SlotShape<2>::STR
-                                : lc <= 4 ? SlotShape<4>::STR : SlotShape<8>::STR);
+    const size_t lds = sizeof(float) * kWavesPerBlock * (size_t)a.slots * SlotShape<LC>::STR;
+    hipLaunchKernelGGL((k_stencils_compact<NWT, LC, true>), dim3(grid), dim3(kBlock), lds, st, a);
+}
+
+template <int NWT>
+static void launch_compact(int lc, const CompactArgs &a, bool lists, int grid, hipStream_t st)
+{
     switch (lc) {
-    case 1: hipLaunchKernelGGL((k_stencils_compact<NWT, 1>), dim3(grid), dim3(kBlock), lds, st, a); break;
-    case 2: hipLaunchKernelGGL((k_stencils_compact<NWT, 2>), dim3(grid), dim3(kBlock), lds, st, a); break;
-    case 3: hipLaunchKernelGGL((k_stencils_compact<NWT, 3>), dim3(grid), dim3(kBlock), lds, st, a); break;
-    case 4: hipLaunchKernelGGL((k_stencils_compact<NWT, 4>), dim3(grid), dim3(kBlock), lds, st, a); break;
-    case 5: hipLaunchKernelGGL((k_stencils_compact<NWT, 5>), dim3(grid), dim3(kBlock), lds, st, a); break;
-    case 6: hipLaunchKernelGGL((k_stencils_compact<NWT, 6>), dim3(grid), dim3(kBlock), lds, st, a); break;
-    case 7: hipLaunchKernelGGL((k_stencils_compact<NWT, 7>), dim3(grid), dim3(kBlock), lds, st, a); break;
-    default: hipLaunchKernelGGL((k_stencils_compact<NWT, 8>), dim3(grid), dim3(kBlock), lds, st, a); break;
+    case 1: launch_compact_lc<NWT, 1>(a, lists, grid, st); break;
+    case 2: launch_compact_lc<NWT, 2>(a, lists, grid, st); break;
+    case 3: launch_compact_lc<NWT, 3>(a, lists, grid, st); break;
+    case 4: launch_compact_lc<NWT, 4>(a, lists, grid, st); break;
+    case 5: launch_compact_lc<NWT, 5>(a, lists, grid, st); break;
+    case 6: launch_compact_lc<NWT, 6>(a, lists, grid, st); break;
+    case 7: launch_compact_lc<NWT, 7>(a, lists, grid, st); break;
+    default: launch_compact_lc<NWT, 8>(a, lists, grid, st); break;
     }
 }
 
@@ -714,9 +724,9 @@ int osdhip_stencil_table_eval(const osdhip_stencil_table *t, const float *src,
             }
             // the kernel computes every weight array of the table; only the
             // requested outputs are written
-            if (t->nw == 1) launch_compact<1>(lc, a, cgrid, st);
-            else if (t->nw == 3) launch_compact<3>(lc, a, cgrid, st);
-            else launch_compact<6>(lc, a, cgrid, st);
+            if (t->nw == 1) launch_compact<1>(lc, a, t->listedSlices > 0, cgrid, st);
+            else if (t->nw == 3) launch_compact<3>(lc, a, t->listedSlices > 0, cgrid, st);
+            else launch_compact<6>(lc, a, t->listedSlices > 0, cgrid, st);
             int rc = last_error();
             if (rc != OSDHIP_OK) return rc;
         }

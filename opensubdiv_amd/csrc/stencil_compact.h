@@ -155,13 +155,13 @@ __device__ __forceinline__ void write_slot(float *p, const float (&x)[LC])
 }
 
 // Sums of an unlisted slice's row: control points gathered from memory, the
-// gathers of two entry groups in flight (one where their values would take
-// too many registers); idx / wp: the slice's indices and weights.
-template <int NWT, int LC, class IP, class P, class S>
+// gathers of GC entry groups in flight; idx / wp: the slice's indices and
+// weights.
+template <int NWT, int LC, int GC, class IP, class P, class S>
 __device__ __forceinline__ void gather_slice(S src, size_t sstride, IP idx, P wp, int W, int lane,
                                              float (&acc)[NWT][LC])
 {
-    constexpr int GC = LC <= 4 ? 2 : 1, N = 4 * GC;
+    constexpr int N = 4 * GC;
     for (int g = 0; 4 * g < W; g += GC) {
         unsigned ii[N];
         float w[GC][NWT][4], v[N][LC];
@@ -198,9 +198,15 @@ __device__ __forceinline__ size_t slice_index_dwords(int W, int U)
     return (size_t)(U >= 0 ? (W + 3) / 4 : W) * kWave;
 }
 
-template <int NWT, int LC>
+// LISTS: some slice of the table lists its control vertices.  The other
+// variant, for one-weight tables of 5 to 8 floats without any list, keeps the
+// gathers of two entry groups in flight, whose registers would cost listed
+// slices their waves (2.1 M rows of 7 floats: 58.9 -> 62.4 us; 500 K rows of
+// 16 random vertices, 7 floats: 56.8 us with two groups, 63.5 with one).
+template <int NWT, int LC, bool LISTS>
 __global__ __launch_bounds__(kBlock) void k_stencils_compact(CompactArgs a)
 {
+    constexpr int GATHER = LC <= 4 || !LISTS ? 2 : 1;   // entry groups gathered at a time
     constexpr int STR = SlotShape<LC>::STR;
     constexpr int GC = NWT == 6 ? 2 : 4;            // entry groups in flight
     // a.slots * STR floats per wave: the table's longest list and the zero slot
@@ -213,7 +219,7 @@ __global__ __launch_bounds__(kBlock) void k_stencils_compact(CompactArgs a)
     if (sl >= a.nslices) return;                     // whole wave idle
     const int s = a.sliceBegin + sl;
     const OSDHIP_CONST SliceDesc &ds = cptr(a.slices)[s];
-    const int W = ds.width, U = ds.nuniq;
+    const int W = ds.width, U = LISTS ? ds.nuniq : -1;
     int row = s * kWave + lane;
     if (a.perm) row = gptr(a.perm)[row];             // wave-uniform branch
     const bool active = row >= a.rowBegin && row < a.rowEnd;
@@ -229,7 +235,7 @@ __global__ __launch_bounds__(kBlock) void k_stencils_compact(CompactArgs a)
 #pragma unroll
         for (int k = 0; k < LC; ++k) acc[w][k] = 0.0f;
 
-    if (U >= 0) {
+    if (LISTS && U >= 0) {
         float *area = lds + wv * a.slots * STR;
         const OSDHIP_GLOBAL int *list = gptr(a.ctrl) + ds.ctrlOff;
         const int G = (W + 3) / 4;
@@ -280,7 +286,7 @@ __global__ __launch_bounds__(kBlock) void k_stencils_compact(CompactArgs a)
                 }
         }
     } else {
-        gather_slice<NWT, LC>(src, sstride, rp, wp, W, lane, acc);
+        gather_slice<NWT, LC, GATHER>(src, sstride, rp, wp, W, lane, acc);
     }
     if (active) {
         const size_t r = (size_t)(row - a.rowBegin);

@@ -190,6 +190,28 @@ def test_batch_wide_listed_slices(L, frames, nlist):
     assert info["listed_slices"] == info["slices"]
 
 
+@pytest.mark.parametrize("layout", [0, 2])
+@pytest.mark.parametrize("L", [4, 5, 7, 8, 11, 16])
+def test_table_without_any_list(hip, layout, L):
+    """A table of scattered rows lists nothing: 5 to 8 floats gather two entry
+    groups at a time, also where a row ends within one of them."""
+    rng = np.random.default_rng(L)
+    n, nsrc = 64 * 3 + 40, 5000
+    sizes = rng.integers(8, 18, size=n).astype(np.int32)
+    sizes[[3, 70]] = 0, 1
+    t = {"sizes": sizes, "offsets": (np.cumsum(sizes) - sizes).astype(np.int32),
+         "indices": rng.integers(0, nsrc, size=int(sizes.sum())).astype(np.int32)}
+    t["weights"] = rng.normal(size=len(t["indices"])).astype(np.float32)
+    table = HipStencilTable.Create(t, layout=layout, order=1 if layout else 0)
+    assert table.layout()["listed_slices"] == 0
+    src = rng.normal(size=(nsrc, L)).astype(np.float32)
+    for start, end in ((0, n), (65, n - 3)):
+        out = empty(n * L)
+        assert table_eval(hip, table.h, dev(src), (0, L, L), [out], [(0, L, L)], start, end) == 0
+        want = oracle.apply_stencils(src, t["sizes"], t["offsets"], t["indices"], t["weights"])
+        np.testing.assert_array_equal(host(out, shape=(n, L))[:end - start], want[start:end])
+
+
 @pytest.mark.parametrize("n,level,far_order", [(7, 4, True), (14, 3, False)])
 def test_large_order_2_tables(hip, n, level, far_order):
     """Tables of 65,536 rows and more under order 2: a level-4 refinement table
