@@ -64,3 +64,18 @@ def test_staged_patches_of_every_point_size(length, frames):
                 assert np.array_equal(o.cpu().numpy().view(np.uint32), w.view(np.uint32)), \
                     (fc, persistent)
     b.close()
+
+
+@pytest.mark.parametrize("layout", [0, 2])
+def test_tuning_times_a_kernel_once(layout):
+    """Phase-A pairs of the same frames per chunk (0: 4) are one kernel: the
+    report gives them one time."""
+    h = compile_mesh(MeshSpec(0, 4, 2, 3, 300, 5), 3)
+    d = DeviceMesh(h, layout=layout, order=0)
+    b = Batch(3, d.stencil_segments())
+    seen = {}
+    for r in b.tune(reps=1)["phase_a"]:
+        seen.setdefault((r["frames"] or 4, r["slices"], r["persistent"]), []).append(r["ms"])
+    assert len(seen) == 18 and all(len(set(ms)) == 1 for ms in seen.values())
+    assert sum(map(len, seen.values())) == (30 if layout == 0 else 36)
+    b.close()
