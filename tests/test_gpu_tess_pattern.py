@@ -27,3 +27,33 @@ def test_pattern_limits(hip, scheme, size, rates):
         for f in {0, nf // 2, nf - 1}:
             assert got[f].tobytes() == np.asarray(want, np.float32).tobytes(), (nf, f)
         assert np.array_equal(got, np.broadcast_to(got[0], got.shape))
+
+
+@pytest.mark.parametrize("rates", [[3, 5, 2, 4], [22], [40, 100], [63], [64]])
+def test_patch_coords_of_many_faces(hip, rates):
+    """PatchCoords of several hundred base faces in shuffled order, from both
+    kernels (64: more than 4,096 points): many blocks, of several faces and of
+    part of them, and a partial last one, equal to
+    osdhip_patch_map_find_faces of the same (face, u, v)."""
+    from gpu_util import dev
+    from opensubdiv_amd import far, meshes
+    from opensubdiv_amd.osd import HipPatchMap
+    m = meshes.cube_sphere(10, seed=4)
+    pt = far.Topology(m).patch_table(2)
+    pm = HipPatchMap(pt.arrays, pt.params)
+    faces = np.random.default_rng(6).permutation(m.nfaces)[:437].astype(np.int32)
+    sizes, base = np.full(m.nfaces, 4, np.int32), np.arange(m.nfaces, dtype=np.int32)
+    r = np.ascontiguousarray(rates, np.int32)
+    nc = hip.osdhip_tess_count(1, 4, len(r), r.ctypes.data)
+    n = len(faces) * nc
+    uv, coords = empty(2 * n), dev(np.full((n, 5), -7, np.int32))
+    dfaces, dsizes, dbase = dev(faces), dev(sizes), dev(base)
+    assert hip.osdhip_tess_coords(1, 4, len(r), r.ctypes.data, len(faces), ptr(uv), ptr(dfaces),
+                                  pm.h, ptr(dsizes), ptr(dbase), len(sizes), ptr(coords),
+                                  stream()) == 0
+    uvh = host(uv, shape=(n, 2)).astype(np.float64)
+    want = dev(np.zeros((n, 5), np.int32))
+    assert pm.FindFaceCoords(n, dev(np.repeat(faces, nc)), dev(np.ascontiguousarray(uvh[:, 0])),
+                             dev(np.ascontiguousarray(uvh[:, 1])), dsizes, dbase, want)
+    assert host(coords, np.int32).tobytes() == host(want, np.int32).tobytes()
+    pm.close()
