@@ -1063,7 +1063,7 @@ def main():
                          "(same topology and recipe) are mapped instead of compiled, the "
                          "rest are compiled and stored")
     ap.add_argument("--table-layout", type=int, default=2, choices=[0, 2],
-                    help="cfg3/cfg4: stencil table layout (0 record slices, 2 locality-ordered)")
+                    help="cfg3/cfg4: stencil table layout (0 Far's row order, 2 locality-ordered)")
     ap.add_argument("--table-order", type=int, default=2, choices=[0, 1, 2],
                     help="cfg3: layout-2 row order (2 by dominant control vertex, 0 then by "
                          "size within row windows, 1 Far's order)")

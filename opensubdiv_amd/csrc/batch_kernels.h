@@ -10,9 +10,11 @@
 //                              vertex buffers phase A completed.
 //
 // Frames are extra right-hand-side columns: a wave loads a table slice's
-// entries once for all frames, and a PatchCoord's basis is evaluated once for all frames.  Element (v, f, k)
-// of a multi-frame buffer lives at base + v * vStride + f * fStride + k, so
-// both frame-major and vertex-major (frames interleaved) layouts work.
+// entries once for all frames (once per chunk of frames where the slice is
+// wider than 16 entries or lists no control vertices), and a PatchCoord's basis
+// is evaluated once for all frames.  Element (v, f, k) of a multi-frame buffer
+// lives at base + v * vStride + f * fStride + k, so both frame-major and
+// vertex-major (frames interleaved) layouts work.
 //
 // Work is cut into items of up to `itemSlices` 64-row slices (phase A) or
 // kBlock coords (phase B).  Static scheduling maps one item to one block;
@@ -205,16 +207,15 @@ __global__ void k_batch_reset(unsigned *counters, int n)
     if (i < n) counters[i] = 0u;
 }
 
-// Next item of this block.  Items are split into kNumXcd contiguous ranges,
-// one per XCD (the hardware places block b on XCD b % 8), so neighbouring
-// slices -- which share control points -- are processed by one XCD and
-// share its L2.  Static: block b takes item xcd_logical_block() once.
-// Persistent: block b claims items from its XCD's range through that
-// range's counter and, when the range is exhausted, from the other ranges in
-// turn; it returns -1 once every range is exhausted.  Must be reached by
-// every thread of the block (it contains __syncthreads).  The result is
-// wave-uniform.
-// claim: two ints of LDS.
+// Next item of this block; neighbouring slices, which share control points, go
+// to one XCD (the hardware places block b on XCD b % 8) and share its L2.
+// Static: block b takes item xcd_logical_block() once, runs of eight items per
+// XCD in turn.  Persistent: the items are split into kNumXcd contiguous ranges,
+// one per XCD; block b claims items from its XCD's range through that range's
+// counter and, when the range is exhausted, from the other ranges in turn; it
+// returns -1 once every range is exhausted.  Must be reached by every thread of
+// the block (it contains __syncthreads).  The result is wave-uniform.  claim:
+// two ints of LDS that nothing else uses while the kernel runs.
 __device__ __forceinline__ int batch_next_item(const BatchArgs &a, int iter, int *claim)
 {
     if (!a.persistent) {
